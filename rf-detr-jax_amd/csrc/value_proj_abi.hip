@@ -4,6 +4,7 @@
 #include "msda_launch.h"
 #include "msda_kernels.h"  // bf16_t
 #include "value_proj_kernels.h"
+#include "value_proj_mfma_kernels.h"
 
 #include <hip/hip_runtime.h>
 
@@ -61,10 +62,85 @@ template <int KIND, typename VT, int BM>
 int launch_g4(const msda::ValueProjParams& p, int grid, hipStream_t st) {
   static std::atomic<int> granted[msda_host::kMaxDevices];  // per instantiation
   auto k = msda::gemm4_kernel<KIND, VT, BM>;
-  const int rc = msda_host::allow_lds(k, msda::G4<BM>::kLdsBytes, granted);
+  using Cfg = msda::G4<BM>;
+  const int rc = msda_host::allow_lds(k, Cfg::kLdsBytes, granted);
   if (rc != MSDA_OK) return rc;
-  hipLaunchKernelGGL(k, dim3(grid), dim3(msda::G4<BM>::kThreads), msda::G4<BM>::kLdsBytes, st, p);
+  hipLaunchKernelGGL(k, dim3(grid), dim3(Cfg::kThreads), Cfg::kLdsBytes, st, p);
   return MSDA_OK;
+}
+
+// The bf16-matrix-unit kernels (value_proj_mfma_kernels.h) need runs of 8 elements of every tensor
+// contiguous and 16-byte aligned: K and D multiples of 8, every tensor they touch on 16 bytes.
+// MSDA_VP_SCALAR and MSDA_VP_BM select the other kernels.
+bool mfma_path(const msda::ValueProjParams& p, const void* a, const void* b) {
+  if (msda_host::env_flag("MSDA_VP_SCALAR") || msda_host::knob("MSDA_VP_BM", 0) != 0) return false;
+  return p.k % 8 == 0 && p.dim % 8 == 0 && aligned_to(p.w, 16) && aligned_to(a, 16) && aligned_to(b, 16);
+}
+
+template <int KIND, typename VT, int CB>
+int launch_rows(const msda::ValueProjParams& p, int lds_limit, int cus, hipStream_t st) {
+  using Cfg = msda::VpRows<KIND, VT, CB>;
+  static std::atomic<int> granted[msda_host::kMaxDevices];  // per instantiation
+  const int64_t m = static_cast<int64_t>(p.batch) * p.seq;
+  const int cols = KIND == msda::kGemmForward ? p.n : p.k, red = KIND == msda::kGemmForward ? p.k : p.n;
+  const int lds = static_cast<int>(Cfg::lds_bytes(red));
+  auto k = msda::vp_rows_kernel<KIND, VT, CB>;
+  const int rc = msda_host::allow_lds(k, lds, granted);
+  if (rc != MSDA_OK) return rc;
+  // workgroups a CU holds at once (LDS, and registers: two waves per SIMD with 256, four with 128)
+  const int resident = std::max(1, std::min(lds_limit / lds, 16 / Cfg::kWaves));
+  const int64_t cgroups = (cols + 32 * CB - 1) / (32 * CB), tiles = (m + 31) / 32;
+  const int64_t rgroups = std::max<int64_t>(1, std::min<int64_t>((tiles + Cfg::kWaves - 1) / Cfg::kWaves, int64_t{cus} * resident / cgroups));
+  hipLaunchKernelGGL(k, dim3(static_cast<unsigned>(cgroups * rgroups)), dim3(Cfg::kThreads), lds, st, p);
+  return MSDA_OK;
+}
+
+template <typename VT, int TILE, bool MASK>
+int launch_gw(const msda::ValueProjParams& p, hipStream_t st) {
+  using Cfg = msda::VpGw<VT, TILE>;
+  static std::atomic<int> granted[msda_host::kMaxDevices];  // per instantiation
+  auto k = msda::vp_gw_kernel<VT, TILE, MASK>;
+  const int rc = msda_host::allow_lds(k, Cfg::kLdsBytes, granted);
+  if (rc != MSDA_OK) return rc;
+  const int64_t tiles = static_cast<int64_t>((p.n + TILE - 1) / TILE) * ((p.k + TILE - 1) / TILE);
+  hipLaunchKernelGGL(k, dim3(static_cast<unsigned>(tiles * p.splits)), dim3(Cfg::kThreads), Cfg::kLdsBytes, st, p);
+  return MSDA_OK;
+}
+
+// The product on the bf16 matrix unit, or MSDA_ERR_UNSUPPORTED (no message) where it would not pay
+// (f32) or one 32-column block of weights does not fit the LDS.
+//   * Rows: two column blocks a workgroup where that leaves four waves (32-row tiles) a CU, else one:
+//     bf16 8 x 576 rows forward 6.4 (one) against 6.6 us, 16 x 6800 42 against 33; four and eight
+//     blocks were slower at every size (52 and 55 us), their LDS leaving room for 8 waves a CU.
+//     f32 takes the path from four waves a CU on: at 1152 rows gemm4_kernel takes 6.5 us against 9.4,
+//     at 4608 13.6 against 13.5 (grad_input 14.1 against 12.0), at 16416 32.9 against 24.3.
+//   * grad_weight: 128-wide tiles (bf16) where they make one workgroup a CU; f32 from 16 slices (4096
+//     rows) on: at 1152 rows 11.8 us against 15.4, at 4608 20.0 against 18.4.
+// MSDA_VP_CB=1 or 2 forces the path and the column blocks.
+template <int KIND, typename VT>
+int launch_mfma(const msda::ValueProjParams& p, hipStream_t st) {
+  int lds = 0, cus = 0;
+  const int rc = msda_host::device_attrs(&lds, &cus);
+  if (rc != MSDA_OK) return rc;
+  constexpr bool bf = sizeof(VT) == 2;
+  const int cb = msda_host::knob("MSDA_VP_CB", 0);
+  if constexpr (KIND == msda::kGemmGradWeight) {
+    if constexpr (bf) {
+      const int64_t t128 = static_cast<int64_t>((p.n + 127) / 128) * ((p.k + 127) / 128) * p.splits;
+      if (t128 >= cus) return p.mask != nullptr ? launch_gw<VT, 128, true>(p, st) : launch_gw<VT, 128, false>(p, st);
+    } else if (p.splits < 16 && cb == 0) {
+      return MSDA_ERR_UNSUPPORTED;
+    }
+    return p.mask != nullptr ? launch_gw<VT, 64, true>(p, st) : launch_gw<VT, 64, false>(p, st);
+  } else {
+    const int cols = KIND == msda::kGemmForward ? p.n : p.k, red = KIND == msda::kGemmForward ? p.k : p.n;
+    const int64_t tiles = (static_cast<int64_t>(p.batch) * p.seq + 31) / 32;
+    if (msda::VpRows<KIND, VT, 2>::lds_bytes(red) <= lds && (cb ? cb == 2 : tiles * ((cols + 63) / 64) >= 4 * int64_t{cus}))
+      return launch_rows<KIND, VT, 2>(p, lds, cus, st);
+    if (msda::VpRows<KIND, VT, 1>::lds_bytes(red) <= lds && (cb ? cb == 1 : bf || tiles * ((cols + 31) / 32) >= 4 * int64_t{cus}))
+      return launch_rows<KIND, VT, 1>(p, lds, cus, st);
+    return MSDA_ERR_UNSUPPORTED;
+  }
 }
 
 // One product: rows x cols outputs (times `splits` slices of the reduction). The 16-byte kernels
@@ -92,7 +168,12 @@ int launch_gemm(const msda::ValueProjParams& p, int64_t rows, int64_t cols, int 
 }
 
 template <int KIND>
-int launch_gemm_dt(const msda::ValueProjParams& p, int64_t rows, int64_t cols, int splits, bool vec, hipStream_t st, const char* what) {
+int launch_gemm_dt(const msda::ValueProjParams& p, int64_t rows, int64_t cols, int splits, bool vec, bool mfma, hipStream_t st,
+                   const char* what) {
+  if (mfma) {
+    const int rc = p.bf16 ? launch_mfma<KIND, msda::bf16_t>(p, st) : launch_mfma<KIND, float>(p, st);
+    if (rc != MSDA_ERR_UNSUPPORTED) return rc != MSDA_OK ? rc : msda_host::check_launch(what);
+  }
   return p.bf16 ? launch_gemm<KIND, msda::bf16_t>(p, rows, cols, splits, vec, st, what)
                 : launch_gemm<KIND, float>(p, rows, cols, splits, vec, st, what);
 }
@@ -127,7 +208,7 @@ int msda_value_proj_fwd(const void* input, int dtype, const float* weight, const
   p.dim_magic = vp_magic(head_dim);
   p.seq_magic = vp_magic(len_in);
   return launch_gemm_dt<msda::kGemmForward>(p, static_cast<int64_t>(batch) * len_in, p.n, 1, vec_path(p, eb, input, nullptr),
-                                            static_cast<hipStream_t>(stream), "value projection forward");
+                                            mfma_path(p, input, value), static_cast<hipStream_t>(stream), "value projection forward");
 }
 
 int64_t msda_value_proj_bwd_workspace_size(int batch, int len_in, int in_features, int n_heads, int head_dim) {
@@ -184,15 +265,16 @@ int msda_value_proj_bwd(const void* input, int dtype, const float* weight, const
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (grad_input != nullptr && m > 0) {
     const bool vec = vec_path(p, eb, grad_value, nullptr);
-    if ((rc = launch_gemm_dt<msda::kGemmGradInput>(p, m, in_features, 1, vec, st, "value projection backward (input)")) != MSDA_OK)
+    if ((rc = launch_gemm_dt<msda::kGemmGradInput>(p, m, in_features, 1, vec, mfma_path(p, grad_value, grad_input),
+                                                    st, "value projection backward (input)")) != MSDA_OK)
       return rc;
   }
   if (want_w) {
     // with no rows the partial sums are zero: the product still runs (every partial is written).
     // The element-wise kernel forms the bias gradient as a column of ones (K + 1 columns); the
     // 16-byte kernel sums dY^T rows instead (K columns).
-    const bool vec = vec_path(p, eb, grad_value, input);
-    if ((rc = launch_gemm_dt<msda::kGemmGradWeight>(p, p.n, static_cast<int64_t>(in_features) + (vec ? 0 : 1), p.splits, vec, st,
+    const bool vec = vec_path(p, eb, grad_value, input), mfma = m > 0 && mfma_path(p, grad_value, input);
+    if ((rc = launch_gemm_dt<msda::kGemmGradWeight>(p, p.n, static_cast<int64_t>(in_features) + (vec ? 0 : 1), p.splits, vec, mfma, st,
                                                      "value projection backward (weight)")) != MSDA_OK)
       return rc;
     const int64_t total = static_cast<int64_t>(p.n) * (in_features + 1);

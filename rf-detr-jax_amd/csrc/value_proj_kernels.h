@@ -735,8 +735,8 @@ __global__ void __launch_bounds__(G4<BM>::kThreads) gemm4_kernel(const ValueProj
   }
 }
 
-// grad_weight [N, K] and grad_bias [N] from the split partial sums, added in split order (the
-// loads of eight splits are issued before their additions).
+// grad_weight [N, K] and grad_bias [N] from the split partial sums, added in a fixed order: eight
+// splits in pairs, then the eights in turn (the loads of eight splits are issued before their additions).
 __global__ void __launch_bounds__(256) wg_reduce_kernel(const ValueProjParams p) {
   const int64_t nk = static_cast<int64_t>(p.n) * p.k, total = nk + p.n;
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < total; i += static_cast<int64_t>(gridDim.x) * 256) {
@@ -749,8 +749,7 @@ __global__ void __launch_bounds__(256) wg_reduce_kernel(const ValueProjParams p)
       float v[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) v[u] = src[(sp + u) * stride];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) s += v[u];
+      s += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
     }
     for (; sp < p.splits; ++sp) s += src[sp * stride];
     if (w) {

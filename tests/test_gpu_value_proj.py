@@ -270,3 +270,75 @@ def test_value_proj_misaligned_tensors(bf16):
     assert_close(_np(gx), rx, tg, "grad_input")
     assert_close(_np(gw), rw, tg, "grad_weight")
     assert_close(_np(gb), rb, tg, "grad_bias")
+
+
+# (batch, rows, K, heads, head_dim): one tile and less; an odd number of 8-element chunks and a column
+# remainder; rows past a 32-row tile that cross batches; more than one batch of reduction steps
+MFMA_SHAPES = [(1, 1, 8, 1, 8), (3, 11, 72, 3, 24), (2, 333, 264, 5, 8), (1, 257, 520, 4, 40), (5, 840, 64, 4, 16)]
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+@pytest.mark.parametrize("blocks", [1, 2])
+@pytest.mark.parametrize("shape", MFMA_SHAPES, ids=str)
+def test_matrix_unit_kernels(tune, shape, blocks, bf16):
+    """The bf16-matrix-unit kernels with one and two column blocks per workgroup (MSDA_VP_CB), with a
+    mask and a bias, against the float64 oracle. f32: the split's terms hold every bit, so the error
+    is that of f32 sums, below sqrt(n) 2^-24 of the 2-norm for n <= 4200 terms in sums of at most 16
+    at a time: 1e-6. bf16 results: one rounding, 2^-8."""
+    b, s, k, h, d = shape
+    _note(f"value_proj matrix unit {shape} blocks={blocks} bf16={bf16}")
+    rng = np.random.default_rng(36)
+    x = rng.standard_normal((b, s, k)).astype(np.float32)
+    w = (rng.standard_normal((h * d, k)) / np.sqrt(k)).astype(np.float32)
+    bias = rng.standard_normal(h * d).astype(np.float32)
+    mask = rng.uniform(0, 1, (b, s)) < 0.2
+    mask[0, 0] = False
+    g = rng.standard_normal((b * h, s, d)).astype(np.float32)
+    if bf16:
+        x, g = bf16_round(x), bf16_round(g)
+    dt = torch.bfloat16 if bf16 else None
+    tune({"MSDA_VP_CB": blocks})
+    out = value_proj_forward(_t(x, dt), _t(w), _t(bias), h, _t(mask))
+    got = [out, *value_proj_backward(_t(x, dt), _t(w), h, _t(g, dt), _t(mask))]
+    torch.cuda.synchronize()
+    x, w, g = x.astype(np.float64), (bf16_round(w) if bf16 else w).astype(np.float64), g.astype(np.float64)
+    bias = (bf16_round(bias) if bf16 else bias).astype(np.float64)
+    want = [VP.value_proj_rows(x, w, bias, h, mask), *VP.value_proj_rows_vjp(x, w, h, g, mask)]
+    for name, a, ref in zip(("value", "grad_input", "grad_weight", "grad_bias"), got, want):
+        tol = 2.0 ** -8 if bf16 and name in ("value", "grad_input") else 1e-6
+        err = np.linalg.norm(_np(a).astype(np.float64) - ref) / np.linalg.norm(ref)
+        assert err <= tol, (name, err)
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+def test_matrix_unit_kernels_nonfinite(tune, bf16):
+    """Infinities, NaN and the largest finite values come out as a plain f32 product has them: in the
+    rows (output, grad_input) and columns (grad_weight) that they reach, and nowhere else."""
+    rng = np.random.default_rng(37)
+    b, s, k, h, d = 2, 200, 64, 4, 16
+    x = rng.integers(-3, 4, (b, s, k)).astype(np.float32)
+    w = rng.integers(1, 4, (h * d, k)).astype(np.float32)
+    g = rng.integers(-3, 4, (b * h, s, d)).astype(np.float32)
+    big = np.finfo(np.float32).max
+    for i, v in enumerate((np.inf, -np.inf, np.nan, big)):
+        x[0, 10 * i + 3], g[1, 9 * i + 5] = 0.0, 0.0
+        x[0, 10 * i + 3, 7 * i], g[1, 9 * i + 5, 3 * i] = v, v
+    w[:, 21] = 0.25  # the largest value times 0.25 is finite
+    w[16 + 9] = 0.25
+    dt = torch.bfloat16 if bf16 else None
+    if bf16:
+        x[0, 33, 21], g[1, 32, 9] = 1.0, 1.0  # bf16 has no such value below infinity
+    tune({"MSDA_VP_CB": 2})
+    got = [value_proj_forward(_t(x, dt), _t(w), None, h), *value_proj_backward(_t(x, dt), _t(w), h, _t(g, dt))[:2]]
+    torch.cuda.synchronize()
+    with np.errstate(all="ignore"):
+        want = [VP.value_proj_rows(x, w, None, h), *VP.value_proj_rows_vjp(x, w, h, g)[:2]]
+        want = [r.astype(np.float32) for r in want]
+    for name, a, ref in zip(("value", "grad_input", "grad_weight"), got, want):
+        a = _np(a)
+        if name == "grad_weight":  # 0 times an infinity is NaN in both; sums of infinities of both signs too
+            assert np.array_equal(np.isfinite(a), np.isfinite(ref)), name
+        fine = np.isfinite(ref)
+        assert np.array_equal(np.isnan(a), np.isnan(ref)), name
+        assert np.array_equal(a[~fine & ~np.isnan(ref)], ref[~fine & ~np.isnan(ref)]), name
+        np.testing.assert_allclose(a[fine], ref[fine], rtol=2.0 ** -8 if bf16 else 1e-6, atol=0)
