@@ -438,15 +438,13 @@ struct AttnWork {
 // V stream through LDS; the running maximum rescales the partial sums. DROP (host: with MASK, the
 // mask may then be null): the dropped weights are zeroed before the product with V, the sum l and
 // the statistics keep every weight, and the output is scaled by drop_scale / l.
-template <typename VT, int D, bool MASK, int RB, bool DROP = false>
-__global__ void __launch_bounds__(64 * RB, D == 32 ? (MASK ? 2 : 3) : (MASK ? 1 : 2)) attn_fwd_kernel(const AttnParams p) {
+template <typename VT, int D, bool MASK, int RB, bool DROP>
+__device__ __forceinline__ void attn_fwd_body(const AttnParams& p, const AttnWork& w, float* at_lds) {
   constexpr int NT = 64 * RB;
   constexpr int LD = D + 8, ND = D / 32;
-  extern __shared__ __align__(16) float at_lds[];
   float* Ks = at_lds;
   float* Vs = at_lds + kAtChunk * LD;
   const int L = p.len, nb = (L + 31) / 32, nchunks = (L + kAtChunk - 1) / kAtChunk;
-  const AttnWork w(p, (nb + RB - 1) / RB);
   const VT* kp = static_cast<const VT*>(p.k) + w.sl.base(p, kAtK);
   const VT* vp = static_cast<const VT*>(p.v) + w.sl.base(p, kAtV);
   const int lane = threadIdx.x & 63, grp = lane >> 5, col = lane & 31;
@@ -505,6 +503,13 @@ __global__ void __launch_bounds__(64 * RB, D == 32 ? (MASK ? 2 : 3) : (MASK ? 1 
       stats[1] = log2f(l);
     }
   }
+}
+
+template <typename VT, int D, bool MASK, int RB, bool DROP = false>
+__global__ void __launch_bounds__(64 * RB, D == 32 ? (MASK ? 2 : 3) : (MASK ? 1 : 2)) attn_fwd_kernel(const AttnParams p) {
+  extern __shared__ __align__(16) float at_lds[];
+  const AttnWork w(p, ((p.len + 31) / 32 + RB - 1) / RB);
+  attn_fwd_body<VT, D, MASK, RB, DROP>(p, w, at_lds);
 }
 
 // Backward, query side: dQ = dS K / sqrt(D) with dS = P (dP - rowsum(dO * O)), dP = dO V^T and P
@@ -1503,23 +1508,24 @@ __global__ void __launch_bounds__(64 * (kAtFusedBlocks + 2), 3) attn_bwd_fused_b
 // into LDS; one phase later key wave 0, which has time to spare, adds the halves and stores the
 // block's rows. Row tiles, dS tiles and the halves are double buffered by phase parity: one
 // barrier per phase.
-constexpr int at_fused_f32_lds_bytes(int nb) { return nb * (32 * 32 * 4 + 2 * 32 * 32 * 4); }  // K copy, two dS tile sets
 
 // element (r, c) of a swizzled f32 tile [32][32]: 16-byte chunk c / 4 of row r at slot (c / 4) ^ ((r / 2) % 8)
 __device__ __forceinline__ int at_f32sw(int r, int c) { return r * 32 + 4 * ((c >> 2) ^ ((r >> 1) & 7)) + (c & 3); }
 
-__global__ void __launch_bounds__(64 * (kAtFusedBlocks + 2), 3) attn_bwd_fused_f32_kernel(const AttnParams p) {
+// Dynamic LDS: 38 KB of row tiles, statistics and dQ halves, then the K copy and the dS tiles.
+constexpr int kAtFusedF32Floats = 2 * (2 * 32 * (32 + 8) + 2 * 32 + 32 + 2 * 16 * 64);
+constexpr int at_fused_f32_lds_bytes(int nb) { return kAtFusedF32Floats * 4 + nb * (32 * 32 * 4 + 2 * 32 * 32 * 4); }
+
+__device__ __forceinline__ void attn_bwd_fused_f32_body(const AttnParams& p, int zh, float* at_lds) {
   constexpr int D = 32, LD = D + 8;
-  __shared__ __align__(16) float Qs[2][32 * LD];  // query rows of the phase's block, by parity
-  __shared__ __align__(16) float Gs[2][32 * LD];  // output-gradient rows
-  __shared__ __align__(16) float Ms[2][2 * 32];   // m, log2 l (rows past L: +inf)
-  __shared__ __align__(16) float Ds[2][32];       // rowsum(dO * O)
-  __shared__ __align__(16) float Xq[2][2][16 * 64];  // the dQ waves' halves of dQ^T (result layout), by parity
-  extern __shared__ __align__(16) float at_lds[];
+  float (*const Qs)[32 * LD] = reinterpret_cast<float (*)[32 * LD]>(at_lds);  // query rows of the phase's block, by parity
+  float (*const Gs)[32 * LD] = Qs + 2;                                        // output-gradient rows
+  float (*const Ms)[2 * 32] = reinterpret_cast<float (*)[2 * 32]>(Gs + 2);    // m, log2 l (rows past L: +inf)
+  float (*const Ds)[32] = reinterpret_cast<float (*)[32]>(Ms + 2);            // rowsum(dO * O)
+  float (*const Xq)[2][16 * 64] = reinterpret_cast<float (*)[2][16 * 64]>(Ds + 2);  // the dQ waves' halves of dQ^T (result layout), by parity
   const int L = p.len, nb = (L + 31) / 32;  // key blocks; also the query blocks (phases)
-  float* Kf = at_lds;                       // [32 nb][32] key rows (0 past L)
+  float* Kf = at_lds + kAtFusedF32Floats;   // [32 nb][32] key rows (0 past L)
   float* St = Kf + 32 * nb * D;             // dS tiles: 1024 floats each, parity, key block
-  const int zh = xcd_logical(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));  // as the bf16 kernel
   const AttnSlice sl(p, zh);
   const float* kp = static_cast<const float*>(p.k) + sl.base(p, kAtK);
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63, grp = lane >> 5, col = lane & 31;

@@ -1,0 +1,698 @@
+// attention_split_kernels.h — gfx950 self-attention of f32 tensors on the 16-bit matrix units, without
+// a mask or dropout: the forward, and the fused backward (head_dim 32, up to 32 kAtFusedBlocks rows).
+//
+// v_mfma_f32_32x32x2_f32 takes 64 cycles for 4096 flops and bounded the f32 kernels
+// (attention_kernels.h). Here every operand, the softmax weights and dS included, is split into
+// 16-bit terms whose products run at 16 times that rate (10 times measured: dense 16-bit MFMAs reach
+// 1.6 PFLOP/s here); sums stay f32.
+//   * Backward: three bf16 terms, each the rounding of what the ones before left, hold all 24
+//     significand bits at any size a bf16 has, so gradients of any range split as well as any other;
+//     six products of terms t and u, t + u <= 2, the five small ones summed before the main one.
+//   * Forward: two f16 terms, h = f16(x) and l = f16(x - h), of values scaled into f16's range; h h +
+//     h l + l h. A scaled value is held to one unit of its 24th bit (exactly in three of four cases).
+//     Half the MFMAs and 2 vector operations per split value instead of 5.5: 76 us where three bf16
+//     terms took 100. Queries are scaled row by row; keys and values by the power of two that puts
+//     the largest element of the first 64 rows at 2^10. What could fall outside f16 then is checked,
+//     not assumed: a key or value beyond 65504, a channel of V whose largest element stays below
+//     2^-1 (its results would lose bits that the f32 kernel keeps), or a query and keys so large that
+//     what their small channels lose could show in the scores (kAtMaxProduct).
+// A workgroup that fails a check, or whose results are not all finite (an infinity leaves the split
+// as NaN), runs the f32 kernel's body instead.
+//
+// Measured (graph replays, f32, before -> after; relative 2-norm against float64 of the output and
+// of grad_q, grad_k, grad_v):
+//   104 slices x 8 heads, 300 x 32: forward 129 -> 76 us, backward 319 -> 238; 3.1e-7 -> 2.1e-7,
+//     4.8, 5.5, 5.5e-7 -> 4.3, 4.1, 4.2e-7
+//   32 x 8, 300 x 32: 44.6 -> 25, 88 -> 69;  2 x 8: 17.1 -> 12, 78 -> 52;  52 x 8, 128 x 32: 15.0 -> 12, 41 -> 37
+//   4 x 8, 600 x 32: forward 32.3 -> 20;  8 x 8, 300 x 64: 30.5 -> 21
+#pragma once
+
+#include <type_traits>
+
+#include "attention_kernels.h"
+
+namespace msda {
+
+typedef _Float16 at_h8 __attribute__((ext_vector_type(8)));
+
+// a and b as packed f16 terms: w = f16(a) | f16(b) << 16 and its remainder r
+__device__ __forceinline__ void at_split2(float a, float b, uint32_t& w, uint32_t& r) {
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  w = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, h2));
+  float ra, rb;  // a - f16(a), exact
+  asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(ra) : "v"(w), "v"(a));
+  asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(rb) : "v"(w), "v"(b));
+  r = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{ra, rb}, h2));
+}
+
+struct AtH8 {  // an operand of eight values: terms h, l
+  at_h8 h, l;
+};
+
+__device__ __forceinline__ AtH8 at_split8(const at_f8& f) {
+  uint32_t w[4], r[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) at_split2(f[2 * i], f[2 * i + 1], w[i], r[i]);
+  return AtH8{__builtin_bit_cast(at_h8, uint4{w[0], w[1], w[2], w[3]}), __builtin_bit_cast(at_h8, uint4{r[0], r[1], r[2], r[3]})};
+}
+
+// result registers i0 .. i0 + 7
+__device__ __forceinline__ AtH8 at_split_regs(const at_f16& v, int i0) {
+  return at_split8(at_f8{v[i0], v[i0 + 1], v[i0 + 2], v[i0 + 3], v[i0 + 4], v[i0 + 5], v[i0 + 6], v[i0 + 7]});
+}
+
+__device__ __forceinline__ void at_mfma(at_f16& c, const at_h8& a, const at_h8& b) {
+  c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+// 2^k with k = 10 - floor(log2 max) (1 for 0; k at most 120), and its inverse
+__device__ __forceinline__ float at_pow2_scale(float max, float& inv) {
+  const int e = static_cast<int>((__float_as_uint(max) >> 23) & 255u);  // biased exponent
+  const int k = max == 0.0f ? 0 : min(137 - e, 120);
+  inv = __uint_as_float(static_cast<uint32_t>(127 - k) << 23);
+  return __uint_as_float(static_cast<uint32_t>(127 + k) << 23);
+}
+
+__device__ __forceinline__ float at_absmax4(const at_f4& v, float m) {
+  return fmaxf(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), m), fmaxf(fabsf(v[2]), fabsf(v[3])));
+}
+
+// Asks the scheduler to follow each of the block's N MFMAs by up to V vector operations: it would
+// issue the dependent MFMAs back to back and the vector work after them.
+template <int N, int V>
+__device__ __forceinline__ void at_interleave() {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x2, V, 0);
+  }
+}
+
+// Term tiles: the rows of a chunk as swizzled f16 tiles [64][D] (at_swo), h then l.
+template <int D>
+__device__ __forceinline__ AtH8 at_tile_row(const uint16_t* X, int stride, int row, int ch) {  // channels ch .. ch + 7
+  const uint16_t* e = X + at_swo<D>(row, ch);
+  return AtH8{__builtin_bit_cast(at_h8, *reinterpret_cast<const uint4*>(e)), __builtin_bit_cast(at_h8, *reinterpret_cast<const uint4*>(e + stride))};
+}
+
+// Operand of X^T for MFMA (nd, s) of at_accum_tr: channel 32 nd + l % 32 at the rows of result
+// registers 8 s .. 8 s + 7, by transposing reads of the term tiles at row x.
+template <int D>
+__device__ __forceinline__ AtH8 at_tile_tr(const uint16_t* X, int stride, int x, int nd, int s, int lane) {
+  const int g = lane >> 4, r = lane & 15, grp = lane >> 5;
+  const int c = 32 * nd + 16 * (g & 1) + 4 * (r & 3), ro = x + 16 * s + 4 * grp + (r >> 2);
+  const int i0 = at_swo<D>(ro, c), i1 = at_swo<D>(ro + 8, c);
+  return AtH8{__builtin_bit_cast(at_h8, at_bf8_of(at_read_tr(X + i0), at_read_tr(X + i1))),
+              __builtin_bit_cast(at_h8, at_bf8_of(at_read_tr(X + stride + i0), at_read_tr(X + stride + i1)))};
+}
+
+// An AtChunk (64 f32 rows in registers) times `scale` as term tiles; rows past L are 0.
+template <int D, int NT>
+__device__ __forceinline__ void at_store_split(const AtChunk<float, D, NT>& ch, float scale, uint16_t* dst, int r0, int L) {
+#pragma unroll
+  for (int u = 0; u < AtChunk<float, D, NT>::NV; ++u) {
+    const int idx = threadIdx.x + NT * u, row = idx / (D / 4), c4 = idx - row * (D / 4);
+    const at_f4 v = ch.v[u] * (r0 + row < L ? scale : 0.0f);
+    uint2 h, l;
+    at_split2(v[0], v[1], h.x, l.x);
+    at_split2(v[2], v[3], h.y, l.y);
+    *reinterpret_cast<uint2*>(&dst[at_swo<D>(row, 4 * c4)]) = h;
+    *reinterpret_cast<uint2*>(&dst[kAtChunk * D + at_swo<D>(row, 4 * c4)]) = l;
+  }
+}
+
+constexpr float kAtF16Max = 65504.0f;
+// What scaling takes from a row's small channels moves a score by at most 2^-30 of max |q| max |k|:
+// f32's own rounding of a score while that product is within this bound (log2 units).
+constexpr float kAtMaxProduct = 256.0f;
+
+template <int D>
+constexpr int at_split_lds_bytes() { return 2 * 2 * 2 * kAtChunk * D * 2 + (4 * D + 4) * 4; }  // key and value term tiles, two buffers; reductions
+static_assert(at_split_lds_bytes<32>() >= at_lds_floats<32>() * 4 && at_split_lds_bytes<64>() >= at_lds_floats<64>() * 4, "the f32 body fits");
+
+// Forward (attn_fwd_kernel's work split and streaming). A workgroup splits each chunk once, into one
+// of two buffers in the shadow of the chunk before's MFMAs. The softmax reference m is moved when a
+// chunk's largest weight would leave [2^3, 2^15] (the first chunk) or exceed 2^15: the weights fit
+// f16, and what they lose below 2^-14 is 2^-28 of the row's largest.
+// Two workgroup-wide MFMA chains per key block pair; vector operations asked between the MFMAs of the
+// scores (10 each: 72 us; left to the compiler 81; 256 registers and two waves per SIMD instead of 168
+// and three: 77).
+template <int D, int RB>
+__global__ void __launch_bounds__(64 * RB, D == 32 ? 3 : 2) attn_fwd_split_kernel(const AttnParams p) {
+  constexpr int NT = 64 * RB, ND = D / 32, TS = kAtChunk * D;  // TS: elements of a term tile
+  extern __shared__ __align__(16) float at_lds[];
+  float* red = at_lds;  // [4][D], [4]
+  uint16_t* Kt = reinterpret_cast<uint16_t*>(at_lds + 4 * D + 4);
+  const int L = p.len, nb = (L + 31) / 32, nchunks = (L + kAtChunk - 1) / kAtChunk;
+  const AttnWork w(p, (nb + RB - 1) / RB);
+  const float* kp = static_cast<const float*>(p.k) + w.sl.base(p, kAtK);
+  const float* vp = static_cast<const float*>(p.v) + w.sl.base(p, kAtV);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, grp = lane >> 5, col = lane & 31;
+  const int qb = w.rc * RB + wave, qi = qb * 32 + col;
+  const bool qv = qi < L;
+  using Chunk = AtChunk<float, D, NT>;
+  Chunk kc, vc;
+  kc.load(kp, p.st[kAtK][3], 0, L);
+  vc.load(vp, p.st[kAtV][3], 0, L);
+  AtH8 qt[D / 16];
+  float iq, qm = 0.0f;  // what the query row was scaled by, inverse; its largest element
+  {
+    const float* qp = static_cast<const float*>(p.q) + w.sl.base(p, kAtQ) + at_row_off(min(qi, L - 1), p.st[kAtQ][3]);
+    at_f4 f[D / 16][2];
+#pragma unroll
+    for (int s = 0; s < D / 16; ++s)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        f[s][u] = *reinterpret_cast<const at_f4*>(qp + 16 * s + 8 * grp + 4 * u);
+        qm = at_absmax4(f[s][u], qm);
+      }
+    qm = at_max_halves(qm);
+    const float sq = at_pow2_scale(qm, iq);
+#pragma unroll
+    for (int s = 0; s < D / 16; ++s) {
+      const at_f4 a = f[s][0] * sq, b = f[s][1] * sq;
+      qt[s] = at_split8(at_f8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]});
+    }
+  }
+  // largest |K| and |V| of the rows a thread stages (V: of its four channels), over the first chunk
+  // for the scales and over all chunks for the checks
+  float kmax = 0.0f;
+  at_f4 vmax = {0.0f, 0.0f, 0.0f, 0.0f};
+  auto track = [&] {
+#pragma unroll
+    for (int u = 0; u < Chunk::NV; ++u) {
+      kmax = at_absmax4(kc.v[u], kmax);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) vmax[e] = fmaxf(vmax[e], fabsf(vc.v[u][e]));
+    }
+  };
+  track();
+  float ik, iv, sk, sv;
+  {
+    float a = kmax, b = fmaxf(fmaxf(vmax[0], vmax[1]), fmaxf(vmax[2], vmax[3]));
+#pragma unroll
+    for (int x = 1; x < 64; x *= 2) {
+      a = fmaxf(a, __shfl_xor(a, x, 64));
+      b = fmaxf(b, __shfl_xor(b, x, 64));
+    }
+    if (lane == 0) {
+      red[wave] = a;
+      red[RB + wave] = b;
+    }
+    __syncthreads();
+    a = red[0];
+    b = red[RB];
+#pragma unroll
+    for (int x = 1; x < RB; ++x) {
+      a = fmaxf(a, red[x]);
+      b = fmaxf(b, red[RB + x]);
+    }
+    sk = at_pow2_scale(a, ik);
+    sv = at_pow2_scale(b, iv);
+  }
+  const float mult = p.scale2 * ik * iq;  // of a product of scaled rows
+  float m = 0.0f, l = 0.0f;               // reference score; sum of the weights
+  at_f16 o[ND], os[ND];                   // O^T: main and small products
+#pragma unroll
+  for (int nd = 0; nd < ND; ++nd) o[nd] = os[nd] = at_zero16();
+  auto stage = [&](int j) {
+    uint16_t* dst = Kt + (j & 1) * 4 * TS;
+    at_store_split<D, NT>(kc, sk, dst, j * kAtChunk, L);
+    at_store_split<D, NT>(vc, sv, dst + 2 * TS, j * kAtChunk, L);
+    kc.load(kp, p.st[kAtK][3], (j + 1) * kAtChunk, L);  // past L: row L - 1 again
+    vc.load(vp, p.st[kAtV][3], (j + 1) * kAtChunk, L);
+  };
+  stage(0);
+  __syncthreads();
+  // One chunk; `last` (a constant): the chunk with the keys past L, which stages nothing.
+  auto chunk = [&](auto last, int j) {
+    constexpr bool LAST = decltype(last)::value;
+    const uint16_t* Kj = Kt + (j & 1) * 4 * TS;
+    const uint16_t* Vj = Kj + 2 * TS;
+    at_f16 s0 = at_zero16(), s1 = at_zero16();  // the chunk's two key blocks
+    {
+      AtH8 a0[D / 16], a1[D / 16];
+#pragma unroll
+      for (int s = 0; s < D / 16; ++s) {
+        a0[s] = at_tile_row<D>(Kj, TS, col, 16 * s + 8 * grp);
+        a1[s] = at_tile_row<D>(Kj, TS, 32 + col, 16 * s + 8 * grp);
+      }
+#pragma unroll
+      for (int s = 0; s < D / 16; ++s) {  // small products first
+        at_mfma(s0, a0[s].h, qt[s].l);
+        at_mfma(s1, a1[s].h, qt[s].l);
+        at_mfma(s0, a0[s].l, qt[s].h);
+        at_mfma(s1, a1[s].l, qt[s].h);
+      }
+#pragma unroll
+      for (int s = 0; s < D / 16; ++s) {
+        at_mfma(s0, a0[s].h, qt[s].h);
+        at_mfma(s1, a1[s].h, qt[s].h);
+      }
+    }
+    if constexpr (!LAST) {
+      track();
+      stage(j + 1);
+      at_interleave<6 * D / 16, 10>();
+    }
+    float bm = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      s0[i] = fmaf(s0[i], mult, -m);
+      s1[i] = fmaf(s1[i], mult, -m);
+      if (LAST) {
+        const int key = j * kAtChunk + 8 * (i >> 2) + 4 * grp + (i & 3);
+        s0[i] = key < L ? s0[i] : -INFINITY;
+        s1[i] = key + 32 < L ? s1[i] : -INFINITY;
+      }
+      bm = at_max3(bm, s0[i], s1[i]);
+    }
+    bm = at_max_halves(bm);  // relative to m; finite: every chunk holds a key below L
+    if (bm > 15.0f || (l == 0.0f && bm < 3.0f)) {
+      bm -= 7.0f;
+      const float alpha = l == 0.0f ? 0.0f : at_exp2(-bm);
+      m += bm;
+      l *= alpha;
+      s0 -= bm;
+      s1 -= bm;
+#pragma unroll
+      for (int nd = 0; nd < ND; ++nd) {
+        o[nd] *= alpha;
+        os[nd] *= alpha;
+      }
+    }
+    float rs = 0.0f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        at_f16& sc = h == 0 ? s0 : s1;
+#pragma unroll
+        for (int i = 8 * s; i < 8 * s + 8; ++i) {
+          sc[i] = at_exp2(sc[i]);
+          rs += sc[i];
+        }
+        const AtH8 b = at_split_regs(sc, 8 * s);
+#pragma unroll
+        for (int nd = 0; nd < ND; ++nd) {  // O^T += V^T P^T
+          const AtH8 a = at_tile_tr<D>(Vj, TS, 32 * h, nd, s, lane);
+          at_mfma(os[nd], a.h, b.l);
+          at_mfma(o[nd], a.h, b.h);
+          at_mfma(os[nd], a.l, b.h);
+        }
+      }
+    l += at_sum_halves(rs);
+  };
+  for (int j = 0; j + 1 < nchunks; ++j) {
+    if (qb < nb) {
+      chunk(std::false_type{}, j);
+    } else {
+      track();
+      stage(j + 1);
+    }
+    __syncthreads();  // chunk j + 1 is staged, and every wave is done with chunk j
+  }
+  if (qb < nb) chunk(std::true_type{}, nchunks - 1);
+  // Channels of V that the scale leaves too small: the largest element of each over the workgroup's
+  // threads (channels 4 c .. 4 c + 3 lie in threads c modulo D / 4)
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+#pragma unroll
+    for (int x = D / 4; x < 64; x *= 2) vmax[e] = fmaxf(vmax[e], __shfl_xor(vmax[e], x, 64));
+  }
+#pragma unroll
+  for (int x = 1; x < 64; x *= 2) kmax = fmaxf(kmax, __shfl_xor(kmax, x, 64));
+  if (lane < D / 4) *reinterpret_cast<at_f4*>(&red[wave * D + 4 * lane]) = vmax;
+  if (lane == 0) red[4 * D + wave] = kmax;
+  __syncthreads();
+#pragma unroll
+  for (int x = 0; x < RB; ++x) kmax = fmaxf(kmax, red[4 * D + x]);
+  bool bad = !(kmax * sk <= kAtF16Max) || (qv && !(qm * kmax * p.scale2 <= kAtMaxProduct));
+  if (static_cast<int>(threadIdx.x) < D) {
+    float v = 0.0f;
+#pragma unroll
+    for (int x = 0; x < RB; ++x) v = fmaxf(v, red[x * D + threadIdx.x]);
+    v *= sv;
+    bad = bad || !(v <= kAtF16Max) || (v != 0.0f && v < 0.5f);
+  }
+  const float inv = iv / l;
+  float z = 0.0f;  // NaN if a result is not finite
+#pragma unroll
+  for (int nd = 0; nd < ND; ++nd) {
+    o[nd] = (o[nd] + os[nd]) * inv;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) z = fmaf(o[nd][i], 0.0f, z);
+  }
+  if (__syncthreads_or(bad || (z != z && qv))) {
+    attn_fwd_body<float, D, false, RB, false>(p, w, at_lds);
+    return;
+  }
+  if (qb < nb) {
+    float* op = static_cast<float*>(p.out) + w.sl.base(p, kAtO);
+#pragma unroll
+    for (int nd = 0; nd < ND; ++nd) at_store_block<float>(op + 32 * nd, p.st[kAtO][3], qb * 32, L, o[nd], 1.0f, at_lds + wave * (at_scratch_bytes<float>() / 4), lane);
+    if (qv && grp == 0) {
+      float* stats = p.stats + (static_cast<int64_t>(w.zh) * L + qi) * 4;
+      stats[0] = m;
+      stats[1] = log2f(l);
+    }
+  }
+}
+
+// ---- backward: three bf16 terms ----------------------------------------------------------------
+constexpr int kAtTerms = 3;
+
+// N f32 values (r, left as what the terms do not hold) as three bf16 terms packed in pairs, largest
+// first. Written on the packed words: element by element the compiler converts twice, once to pack
+// and once to subtract.
+template <int N>
+__device__ __forceinline__ void at_split(float (&r)[N], uint32_t (&t)[kAtTerms][N / 2]) {
+  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+  typedef float f2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int u = 0; u < kAtTerms; ++u)
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+      t[u][i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{r[2 * i], r[2 * i + 1]}, bf2));
+      if (u + 1 < kAtTerms) {
+        r[2 * i] -= __uint_as_float(t[u][i] << 16);
+        r[2 * i + 1] -= __uint_as_float(t[u][i] & 0xffff0000u);
+      }
+    }
+}
+
+__device__ __forceinline__ void at_split8(const at_f8& f, at_bf8 (&t)[kAtTerms]) {
+  float r[8] = {f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7]};
+  uint32_t w[kAtTerms][4];
+  at_split(r, w);
+#pragma unroll
+  for (int u = 0; u < kAtTerms; ++u) t[u] = __builtin_bit_cast(at_bf8, uint4{w[u][0], w[u][1], w[u][2], w[u][3]});
+}
+
+__device__ __forceinline__ void at_split4(const at_f4& f, uint2 (&t)[kAtTerms]) {
+  float r[4] = {f[0], f[1], f[2], f[3]};
+  uint32_t w[kAtTerms][2];
+  at_split(r, w);
+#pragma unroll
+  for (int u = 0; u < kAtTerms; ++u) t[u] = uint2{w[u][0], w[u][1]};
+}
+
+// result registers i0 .. i0 + 7
+__device__ __forceinline__ void at_split_regs(const at_f16& v, int i0, at_bf8 (&t)[kAtTerms]) {
+  at_split8(at_f8{v[i0], v[i0 + 1], v[i0 + 2], v[i0 + 3], v[i0 + 4], v[i0 + 5], v[i0 + 6], v[i0 + 7]}, t);
+}
+
+// channels 16 s + 8 grp .. + 7 of a 16-byte aligned f32 row, s < D / 16
+template <int D>
+__device__ __forceinline__ void at_row_split(at_bf8 (&t)[D / 16][kAtTerms], const float* row, int grp) {
+#pragma unroll
+  for (int s = 0; s < D / 16; ++s) {
+    const at_f4 a = *reinterpret_cast<const at_f4*>(row + 16 * s + 8 * grp), b = *reinterpret_cast<const at_f4*>(row + 16 * s + 8 * grp + 4);
+    at_split8(at_f8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}, t[s]);
+  }
+}
+
+__device__ __forceinline__ void at_mfma(at_f16& c, const at_bf8& a, const at_bf8& b) {
+  c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// small += the five small term products, smallest first
+__device__ __forceinline__ void at_mfma_small(at_f16& small, const at_bf8 (&a)[kAtTerms], const at_bf8 (&b)[kAtTerms]) {
+  at_mfma(small, a[0], b[2]);
+  at_mfma(small, a[1], b[1]);
+  at_mfma(small, a[2], b[0]);
+  at_mfma(small, a[0], b[1]);
+  at_mfma(small, a[1], b[0]);
+}
+
+// Result-layout products of the 32 rows at row x of the swizzled term tiles X (`stride` elements
+// apart) and the lane's register row: the small products of all channels first, then the main ones.
+template <int D>
+__device__ __forceinline__ at_f16 at_scores_split(const uint16_t* X, int stride, int x, const at_bf8 (&r)[D / 16][kAtTerms], int col, int grp) {
+  at_bf8 a[D / 16][kAtTerms];
+#pragma unroll
+  for (int s = 0; s < D / 16; ++s)
+#pragma unroll
+    for (int u = 0; u < kAtTerms; ++u)
+      a[s][u] = __builtin_bit_cast(at_bf8, *reinterpret_cast<const uint4*>(&X[u * stride + at_swo<D>(x + col, 16 * s + 8 * grp)]));
+  at_f16 acc = at_zero16();
+#pragma unroll
+  for (int s = 0; s < D / 16; ++s) at_mfma_small(acc, a[s], r[s]);
+#pragma unroll
+  for (int s = 0; s < D / 16; ++s) at_mfma(acc, a[s][0], r[s][0]);
+  return acc;
+}
+
+// Operand of X^T for MFMA (nd, s) of at_accum_tr: channel 32 nd + l % 32 at the rows of result
+// registers 8 s .. 8 s + 7, by transposing reads of the term tiles at row x.
+template <int D>
+__device__ __forceinline__ void at_operand_tr(at_bf8 (&a)[kAtTerms], const uint16_t* X, int stride, int x, int nd, int s, int lane) {
+  const int g = lane >> 4, r = lane & 15, grp = lane >> 5;
+  const int c = 32 * nd + 16 * (g & 1) + 4 * (r & 3), ro = x + 16 * s + 4 * grp + (r >> 2);
+#pragma unroll
+  for (int u = 0; u < kAtTerms; ++u) a[u] = at_bf8_of(at_read_tr(X + u * stride + at_swo<D>(ro, c)), at_read_tr(X + u * stride + at_swo<D>(ro + 8, c)));
+}
+
+// Fused backward: one workgroup per (slice, head), one phase per 32-row query block. Key waves (one
+// per key block, K and V terms in registers) form S, dP, P and dS of their block against the
+// phase's query block, write dS as three term tiles [32 keys][32 queries], and accumulate dV and dK.
+// The two dQ waves stage the query rows (Q and dO terms, rowsum(dO * O)) one block ahead and form
+// 16 channels each of the previous block's dQ^T = K^T dS^T over all key blocks
+// (v_mfma_f32_16x16x32_bf16, one key block per product), straight to memory. The dS tiles of one
+// block fill 61 KB at 320 rows, as much as the key terms, so there is one set of them: between the
+// two barriers of a phase the key waves write their tiles, and dV, dK and the next block's scores
+// overlap the dQ waves' products. The query rows have three buffers: the dQ waves write one while
+// key waves may still read the two before it.
+constexpr int kAtSplitRow = 32 * 32;  // elements of one term of a 32-row tile
+constexpr int at_fused_split_lds_bytes(int nb) {
+  return 3 * (2 * kAtTerms * kAtSplitRow * 2 + 3 * 32 * 4) + 16 + 2 * nb * kAtTerms * kAtSplitRow * 2;
+}
+
+__global__ void __launch_bounds__(64 * (kAtFusedBlocks + 2), 3) attn_bwd_fused_split_kernel(const AttnParams p) {
+  constexpr int D = 32, TR = kAtSplitRow;
+  extern __shared__ __align__(16) float at_lds[];
+  const int L = p.len, nb = (L + 31) / 32;
+  float* Ms = at_lds;                     // [3][32][2]: m, log2 l (rows past L: +inf)
+  float* Ds = Ms + 3 * 64;                // [3][32]: rowsum(dO * O)
+  int* bad = reinterpret_cast<int*>(Ds + 3 * 32);  // a result is not finite
+  uint16_t* Qt = reinterpret_cast<uint16_t*>(bad + 4);  // [3][term][32][32]
+  uint16_t* Gt = Qt + 3 * kAtTerms * TR;
+  uint16_t* Kt = Gt + 3 * kAtTerms * TR;  // [term][32 nb][32] (0 past L)
+  uint16_t* St = Kt + kAtTerms * nb * TR;  // [key block][term][32][32]
+  const int zh = xcd_logical(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));  // as the bf16 kernel
+  const AttnSlice sl(p, zh);
+  const float* kp = static_cast<const float*>(p.k) + sl.base(p, kAtK);
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63, grp = lane >> 5, col = lane & 31;
+  if (t == 0) *bad = 0;
+  float z = 0.0f;  // NaN if a result of this lane is not finite
+  if (wave < nb) {  // key block kb = wave (uniform per wave)
+    const int kb = wave, kcl = min(kb * 32 + col, L - 1);
+    at_bf8 kt[D / 16][kAtTerms], vt[D / 16][kAtTerms];
+    {
+      at_f4 kc[4];  // the block's rows of the key copy: row 8 u + lane / 8, channels 4 (lane % 8) .. + 3
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int row = kb * 32 + 8 * u + (lane >> 3);
+        kc[u] = row < L ? *reinterpret_cast<const at_f4*>(kp + at_row_off(row, p.st[kAtK][3]) + 4 * (lane & 7)) : at_f4{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+      at_row_split<D>(kt, kp + at_row_off(kcl, p.st[kAtK][3]), grp);
+      at_row_split<D>(vt, static_cast<const float*>(p.v) + sl.base(p, kAtV) + at_row_off(kcl, p.st[kAtV][3]), grp);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        uint2 x[kAtTerms];
+        at_split4(kc[u], x);
+#pragma unroll
+        for (int q = 0; q < kAtTerms; ++q) *reinterpret_cast<uint2*>(&Kt[q * nb * TR + at_swo<D>(kb * 32 + 8 * u + (lane >> 3), 4 * (lane & 7))]) = x[q];
+      }
+    }
+    at_f16 dk = at_zero16(), dv = at_zero16();
+    __syncthreads();  // query block 0 staged, key terms written
+    for (int j = 0, b = 0; j < nb; ++j, b = b == 2 ? 0 : b + 1) {
+      const uint16_t* Qb = Qt + b * kAtTerms * TR;
+      const uint16_t* Gb = Gt + b * kAtTerms * TR;
+      if (kb == 0 && lane < 32 && j * 32 + lane < L)  // rowsum(dO * O) into the statistics (their entry 2)
+        p.stats[(static_cast<int64_t>(zh) * L + j * 32 + lane) * 4 + 2] = Ds[32 * b + lane];
+      at_f16 s = at_scores_split<D>(Qb, TR, 0, kt, col, grp);         // S = Q K^T
+      const at_f16 dp = at_scores_split<D>(Gb, TR, 0, vt, col, grp);  // dP = dO V^T
+      at_f16 pw;
+#pragma unroll
+      for (int c4 = 0; c4 < 4; ++c4) {
+        const int ql = 8 * c4 + 4 * grp;
+        const at_f4 ms0 = *reinterpret_cast<const at_f4*>(&Ms[64 * b + 2 * ql]), ms1 = *reinterpret_cast<const at_f4*>(&Ms[64 * b + 2 * ql + 4]);
+        const at_f4 dd = *reinterpret_cast<const at_f4*>(&Ds[32 * b + ql]);
+        const float mq[4] = {ms0[0], ms0[2], ms1[0], ms1[2]}, lq[4] = {ms0[1], ms0[3], ms1[1], ms1[3]};
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          const int i = 4 * c4 + jj;
+          // a lane past L holds the clamped last key: finite weights, and its rows of the key copy
+          // are 0, so it adds nothing to dQ; rows past L have m = +inf: weight 0
+          pw[i] = at_exp2(fmaf(s[i], p.scale2, -mq[jj]) - lq[jj]);
+          s[i] = pw[i] * (dp[i] - dd[jj]);  // dS
+        }
+      }
+      at_bf8 ds[2][kAtTerms];
+      at_split_regs(s, 0, ds[0]);
+      at_split_regs(s, 8, ds[1]);
+      __syncthreads();  // the dQ waves are done with the previous block's tiles
+      uint16_t* T = St + kb * kAtTerms * TR;  // row = key (this lane's col), columns = the block's queries
+#pragma unroll
+      for (int u = 0; u < kAtTerms; ++u)
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2) {
+          const uint4 x = __builtin_bit_cast(uint4, ds[s2][u]);
+          *reinterpret_cast<uint2*>(&T[u * TR + at_swo<D>(col, 16 * s2 + 4 * grp)]) = uint2{x.x, x.y};
+          *reinterpret_cast<uint2*>(&T[u * TR + at_swo<D>(col, 16 * s2 + 8 + 4 * grp)]) = uint2{x.z, x.w};
+        }
+      __syncthreads();  // the block's tiles are written
+      // dK^T += Q^T dS and dV^T += dO^T P: the block's sums by themselves, then added
+      {
+        at_f16 acc = at_zero16();
+        at_bf8 a0[kAtTerms], a1[kAtTerms];
+        at_operand_tr<D>(a0, Qb, TR, 0, 0, 0, lane);
+        at_operand_tr<D>(a1, Qb, TR, 0, 0, 1, lane);
+        at_mfma_small(acc, a0, ds[0]);
+        at_mfma_small(acc, a1, ds[1]);
+        at_mfma(acc, a0[0], ds[0][0]);
+        at_mfma(acc, a1[0], ds[1][0]);
+        dk += acc;
+      }
+      {
+        at_f16 acc = at_zero16();
+        at_bf8 pt[2][kAtTerms], a0[kAtTerms], a1[kAtTerms];
+        at_split_regs(pw, 0, pt[0]);
+        at_split_regs(pw, 8, pt[1]);
+        at_operand_tr<D>(a0, Gb, TR, 0, 0, 0, lane);
+        at_operand_tr<D>(a1, Gb, TR, 0, 0, 1, lane);
+        at_mfma_small(acc, a0, pt[0]);
+        at_mfma_small(acc, a1, pt[1]);
+        at_mfma(acc, a0[0], pt[0][0]);
+        at_mfma(acc, a1[0], pt[1][0]);
+        dv += acc;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) z = fmaf(dk[i], 0.0f, fmaf(dv[i], 0.0f, z));
+    if (z != z) *bad = 1;
+    __syncthreads();  // the dQ waves are done with the tiles and the key terms
+    if (*bad == 0) {
+      float* sc = reinterpret_cast<float*>(Kt) + kb * (at_scratch_bytes<float>() / 4);  // output scratch
+      if (p.gk != nullptr) at_store_block<float>(static_cast<float*>(p.gk) + sl.base(p, kAtGK), p.st[kAtGK][3], kb * 32, L, dk, p.scale, sc, lane);
+      if (p.gv != nullptr) at_store_block<float>(static_cast<float*>(p.gv) + sl.base(p, kAtGV), p.st[kAtGV][3], kb * 32, L, dv, 1.0f, sc, lane);
+    }
+  } else {
+    // The two dQ waves. Staging: thread tq holds row tq / 4 of a block, channels 8 (tq % 4) .. + 7.
+    const int tq = t - 64 * nb, ch0 = 16 * (tq >> 6);  // this wave's channels of dQ
+    const float* qp = static_cast<const float*>(p.q) + sl.base(p, kAtQ);
+    const float* gop = static_cast<const float*>(p.go) + sl.base(p, kAtGO);
+    const float* opp = static_cast<const float*>(p.o) + sl.base(p, kAtO);
+    const float* stats = p.stats + static_cast<int64_t>(zh) * L * 4;
+    const int srow = tq >> 2, sq4 = tq & 3;
+    at_f8 qv, gv, ov;
+    float2 sq = {0.0f, 0.0f};  // m, log2 l
+    auto ld8 = [](const float* e) {
+      const at_f4 a = *reinterpret_cast<const at_f4*>(e), b = *reinterpret_cast<const at_f4*>(e + 4);
+      return at_f8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    };
+    auto prefetch = [&](int r0) {
+      const int r = min(r0 + srow, L - 1);
+      qv = ld8(qp + at_row_off(r, p.st[kAtQ][3]) + 8 * sq4);
+      gv = ld8(gop + at_row_off(r, p.st[kAtGO][3]) + 8 * sq4);
+      ov = ld8(opp + at_row_off(r, p.st[kAtO][3]) + 8 * sq4);
+      if (sq4 == 0) sq = *reinterpret_cast<const float2*>(&stats[4 * r]);
+    };
+    auto stage = [&](int r0, int b) {
+      const bool in = r0 + srow < L;
+      float dd = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) dd += gv[e] * ov[e];
+      const at_f8 zero = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+      at_bf8 qs[kAtTerms], gs[kAtTerms];
+      at_split8(in ? qv : zero, qs);
+      at_split8(in ? gv : zero, gs);
+#pragma unroll
+      for (int u = 0; u < kAtTerms; ++u) {
+        *reinterpret_cast<uint4*>(&Qt[(b * kAtTerms + u) * TR + at_swo<D>(srow, 8 * sq4)]) = __builtin_bit_cast(uint4, qs[u]);
+        *reinterpret_cast<uint4*>(&Gt[(b * kAtTerms + u) * TR + at_swo<D>(srow, 8 * sq4)]) = __builtin_bit_cast(uint4, gs[u]);
+      }
+      // the row's four quarters: neighbouring lanes (DPP quad_perm [1, 0, 3, 2], then [2, 3, 0, 1])
+      dd += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(dd), 0xB1, 0xF, 0xF, false));
+      dd += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(dd), 0x4E, 0xF, 0xF, false));
+      if (sq4 == 0) {
+        Ms[64 * b + 2 * srow] = in ? sq.x : INFINITY;
+        Ms[64 * b + 2 * srow + 1] = in ? sq.y : 0.0f;
+        Ds[32 * b + srow] = in ? dd : 0.0f;
+      }
+    };
+    float* gqp = static_cast<float*>(p.gq) + sl.base(p, kAtGQ);
+    const bool gq16 = (reinterpret_cast<uintptr_t>(gqp) & 15) == 0 && (p.st[kAtGQ][3] & 3) == 0;
+    const int g = lane >> 4, i16 = lane & 15;
+    // dQ^T of query block jq, channels ch0 .. + 15: lane l of v_mfma_f32_16x16x32_bf16 supplies row
+    // (or column) l % 16 at reduction slots 8 (l / 16) .. + 7, here the keys of a block, each half of
+    // them by one transposing read; its results are channels ch0 + 4 (l / 16) .. + 3 of query l % 16
+    auto dq = [&](int jq) {
+      at_f4 acc[2], small[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) acc[h] = small[h] = at_f4{0.0f, 0.0f, 0.0f, 0.0f};
+      const int ro = 8 * g + (i16 >> 2), co = 4 * (i16 & 3);
+      for (int kb = 0; kb < nb; ++kb) {
+        at_bf8 a[kAtTerms], x[2][kAtTerms];
+#pragma unroll
+        for (int u = 0; u < kAtTerms; ++u) {
+          const uint16_t* K = Kt + (u * nb + kb) * TR;
+          const uint16_t* T = St + (kb * kAtTerms + u) * TR;
+          a[u] = at_bf8_of(at_read_tr(K + at_swo<D>(ro, ch0 + co)), at_read_tr(K + at_swo<D>(ro + 4, ch0 + co)));
+#pragma unroll
+          for (int h = 0; h < 2; ++h) x[h][u] = at_bf8_of(at_read_tr(T + at_swo<D>(ro, 16 * h + co)), at_read_tr(T + at_swo<D>(ro + 4, 16 * h + co)));
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          auto mm = [&](at_f4& c, int u, int v) { c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], x[h][v], c, 0, 0, 0); };
+          mm(small[h], 0, 2);
+          mm(small[h], 1, 1);
+          mm(small[h], 2, 0);
+          mm(small[h], 0, 1);
+          mm(small[h], 1, 0);
+          mm(acc[h], 0, 0);
+        }
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int q = 32 * jq + 16 * h + i16;
+        const at_f4 v = (acc[h] + small[h]) * p.scale;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) z = q < L ? fmaf(v[e], 0.0f, z) : z;
+        if (q >= L) continue;
+        float* dst = gqp + at_row_off(q, p.st[kAtGQ][3]) + ch0 + 4 * g;
+        if (gq16) {
+          *reinterpret_cast<at_f4*>(dst) = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) dst[e] = v[e];
+        }
+      }
+    };
+    prefetch(0);
+    stage(0, 0);
+    if (nb > 1) prefetch(32);
+    __syncthreads();  // query block 0 staged, key terms written
+    for (int j = 0, b = 1; j < nb; ++j, b = b == 2 ? 0 : b + 1) {
+      if (j > 0) dq(j - 1);
+      if (j + 1 < nb) {  // read from the second barrier of phase j on
+        stage((j + 1) * 32, b);
+        if (j + 2 < nb) prefetch((j + 2) * 32);
+      }
+      __syncthreads();
+      __syncthreads();
+    }
+    dq(nb - 1);
+    if (z != z) *bad = 1;
+    __syncthreads();
+  }
+  if (*bad != 0) {  // the same for every thread: read after the last barrier
+    __syncthreads();  // every wave has read the flag: the f32 body takes the LDS over
+    attn_bwd_fused_f32_body(p, zh, at_lds);
+  }
+}
+
+}  // namespace msda

@@ -590,3 +590,83 @@ def test_dropout_module_training_and_eval():
     q, k, v = (torch.randn(1, 2, 33, 32, device=_dev()) for _ in range(3))
     assert torch.equal(scaled_dot_product_attention(q, k, v, dropout=0.0, seed=3), scaled_dot_product_attention(q, k, v))
     assert not scaled_dot_product_attention(q, k, v, dropout=1.0).any()
+
+
+SPLIT_RANGES = ["tiny", "large", "late_keys", "small_channels", "zero_first", "row_range"]
+
+
+def _split_inputs(kind, shape):
+    rng = np.random.default_rng(61)
+    b, h, length, d = shape
+    q, k, v, g = (rng.standard_normal(shape).astype(np.float32) for _ in range(4))
+    if kind == "tiny":  # far below f16's range, some values below 2^-126
+        k, v, g = k * np.float32(1e-32), v * np.float32(1e-36), g * np.float32(1e-30)
+    elif kind == "large":  # far above it
+        q, k, v, g = q * np.float32(1e-12), k * np.float32(1e12), v * np.float32(1e30), g * np.float32(1e-20)
+    elif kind == "late_keys":  # rows past the first 64 overflow the scale taken from those
+        first = min(64, length // 2)
+        q, k[:, :, first:], v[:, :, first:] = q / np.float32(200), k[:, :, first:] * np.float32(200), v[:, :, first:] * np.float32(200)
+    elif kind == "small_channels":  # channels that the shared scale would leave without their low bits
+        v = v * np.where(np.arange(d) % 3 == 0, 1e-7, 1.0).astype(np.float32)
+    elif kind == "zero_first":  # nothing to take a scale from
+        k[:, :, :64], v[:, :, :64] = 0.0, 0.0
+    else:  # rows of very different sizes
+        size = 10.0 ** rng.uniform(-8, 0, (b, h, length, 1))
+        q, g = (q * size).astype(np.float32), (g * size[:, :, ::-1]).astype(np.float32)
+    return q, k, v, g
+
+
+@pytest.mark.parametrize("kind", SPLIT_RANGES)
+@pytest.mark.parametrize("shape", [(2, 2, 300, 32), (1, 3, 65, 64), (2, 1, 33, 32)], ids=str)
+def test_split_operands_of_any_size(shape, kind):
+    """f32 operands are split into 16-bit terms: sizes and spreads that 16 bits do not cover, against the
+    float64 oracle. Errors are relative to the 2-norm of each output channel and of each grad_q row
+    (a shared scale must not cost the small ones their bits): a few hundred terms at f32's 2^-24 and
+    the rounding of the scores, 8e-6."""
+    _note(f"sdpa split operands {kind} {shape}")
+    q, k, v, g = _split_inputs(kind, shape)
+    tq, tk, tv = (_t(x).requires_grad_(True) for x in (q, k, v))
+    out = scaled_dot_product_attention(tq, tk, tv)
+    out.backward(_t(g))
+    torch.cuda.synchronize()
+
+    def err(got, want, axes):
+        got, want = got.detach().double().cpu().numpy(), np.asarray(want, np.float64)
+        n = np.sqrt((want ** 2).sum(axes))
+        # below 2^-120 f32 itself has few bits left
+        ok = n > 2.0 ** -120
+        return float((np.sqrt(((got - want) ** 2).sum(axes))[ok] / n[ok]).max()) if ok.any() else 0.0
+
+    want = AT.sdpa(q, k, v)
+    gq, gk, gv = AT.sdpa_vjp(q, k, v, g)
+    _note(f"errors: {err(out, want, 2):.2g} {err(tq.grad, gq, 3):.2g} {err(tk.grad, gk, (2, 3)):.2g} {err(tv.grad, gv, (2, 3)):.2g}")
+    assert err(out, want, 2) <= 8e-6, "out"
+    assert err(tv.grad, gv, (2, 3)) <= 8e-6, "grad_v"
+    if kind != "tiny":  # grad_q and grad_k are products of what is tiny: below f32's range
+        assert err(tq.grad, gq, 3) <= 1e-4, "grad_q"  # a row's terms cancel: dP - rowsum(dO O)
+        assert err(tk.grad, gk, (2, 3)) <= 1e-5, "grad_k"
+
+
+@pytest.mark.parametrize("where", ["q", "k", "v", "g"])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3.4e38], ids=str)
+def test_split_operands_nonfinite(tune, where, value):
+    """An infinity, a NaN or a value that 16 bits round to infinity gives what the f32 kernels give: the
+    forward with a mask that blocks nothing, the backward in its two-kernel form."""
+    rng = np.random.default_rng(62)
+    x = {n: rng.standard_normal((2, 2, 96, 32)).astype(np.float32) for n in "qkvg"}
+    x[where][0, 1, 70, 5] = value
+    if value == 3.4e38:  # finite scores: its partner is small
+        x[{"q": "k", "k": "q", "v": "g", "g": "v"}[where]][0, 1, :, 5] *= 1e-36
+    got, want = [], []
+    for res, mask, fused in ((got, None, 1), (want, _t(np.zeros((96, 96), bool)), 0)):
+        tune({"MSDA_ATTN_FUSED": fused})
+        t = {n: _t(x[n]).requires_grad_(True) for n in "qkv"}
+        out = scaled_dot_product_attention(t["q"], t["k"], t["v"], mask)
+        res += [out, *torch.autograd.grad(out, list(t.values()), _t(x["g"]))]
+    torch.cuda.synchronize()
+    for name, a, b in zip(("out", "grad_q", "grad_k", "grad_v"), got, want):
+        a, b = _np(a).astype(np.float64), _np(b).astype(np.float64)
+        fine = np.isfinite(b)
+        assert np.array_equal(fine, np.isfinite(a)), name
+        assert np.array_equal(np.isnan(a), np.isnan(b)), name
+        np.testing.assert_allclose(a[fine], b[fine], rtol=1e-4, atol=1e-5 * max(1.0, np.abs(b[fine]).max()))
