@@ -8,10 +8,13 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import importlib.util
 import os
 import threading
 
-from .build import LIB_PATH
+import torch
+
+from .build import BINDING_PATH, LIB_PATH
 
 DTYPE_F32 = 0
 DTYPE_BF16 = 1
@@ -68,6 +71,7 @@ SAMPLE_NEAREST = 1
 
 _lock = threading.Lock()
 _lib = None
+_binding = None
 
 
 class MsdaError(RuntimeError):
@@ -100,6 +104,27 @@ def lib(path: str | None = None) -> ctypes.CDLL:
         if path is None:
             _lib = handle
         return handle
+
+
+def binding():
+    """Load (once) and return the torch binding: the differentiable ops as C++ autograd functions over
+    the library's C ABI, each returning None for a call that the Python path has to take."""
+    global _binding
+    if _binding is not None:
+        return _binding
+    handle = lib()
+    with _lock:
+        if _binding is not None:
+            return _binding
+        if not os.path.exists(BINDING_PATH):
+            raise RuntimeError(f"torch binding not found at {BINDING_PATH}; build it with __graft_entry__.build()")
+        spec = importlib.util.spec_from_file_location("rfdetr_jax_amd._torch_binding", BINDING_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        address = {name: ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in SIGNATURES}
+        module.bind(address, check, torch.nn.Parameter)
+        _binding = module
+        return _binding
 
 
 def check(rc: int) -> None:

@@ -184,6 +184,10 @@ def scaled_dot_product_attention(q, k, v, mask=None, dropout=0.0, seed=None):
     drop = _dropout_args(dropout, seed)
     if drop == "all":
         return torch.zeros(q.shape, dtype=q.dtype, device=q.device)
+    if mask is None and drop is None:
+        out = _native.binding().attention(q, k, v, 0, 1)
+        if out is not None:
+            return out
     b, h, length, d = q.shape
     return _AttentionFunction.apply(q, k, v, mask, _Layout(b, 1, h, length, d), False, drop)
 
@@ -203,6 +207,10 @@ def grouped_attention(q, k, v, num_heads, groups=1, mask=None, dropout=0.0, seed
     drop = _dropout_args(dropout, seed)
     if drop == "all":
         return torch.zeros(q.shape, dtype=q.dtype, device=q.device)
+    if mask is None and drop is None and type(num_heads) is int and type(groups) is int and num_heads > 0:
+        out = _native.binding().attention(q, k, v, num_heads, groups)
+        if out is not None:
+            return out
     return _AttentionFunction.apply(q, k, v, mask, _Layout(b, groups, num_heads, total // groups, c // num_heads), True, drop)
 
 

@@ -1,4 +1,4 @@
-"""Build the gfx950 HIP library ``libmsda_gfx950.so`` in-tree with hipcc.
+"""Build the gfx950 HIP library ``libmsda_gfx950.so`` (hipcc) and the torch binding over it (g++) in-tree.
 
 ``python -m rfdetr_jax_amd.build`` (with ``rf-detr-jax_amd/`` on ``sys.path``) or
 ``__graft_entry__.build()`` runs it. The library is placed next to this file, where
@@ -20,6 +20,7 @@ CSRC = os.path.join(ROOT, "csrc")
 INCLUDE = os.path.join(REPO, "include")
 LIB_NAME = "libmsda_gfx950.so"
 LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
+BINDING_PATH = os.path.join(PKG_DIR, "_torch_binding.so")
 # The C ABI, and the kernel instantiations split by value dtype and direction so they compile in
 # parallel.
 SOURCES = [os.path.join(CSRC, f) for f in ("msda_abi.hip", "msda_fwd_f32.hip", "msda_fwd_bf16.hip", "msda_bwd_f32.hip",
@@ -61,8 +62,26 @@ def _run(cmd: list[str], verbose: bool) -> None:
         sys.stderr.write(proc.stderr)
 
 
+def binding_command(out: str) -> list[str]:
+    """g++ on csrc/torch_binding.cpp against this torch: host code only, the kernel library not linked."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    system = [f for d in (*include_paths(), os.path.join(rocm, "include")) for f in ("-isystem", d)]
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *system, "-I", sysconfig.get_paths()["include"],
+            "-I", INCLUDE, os.path.join(CSRC, "torch_binding.cpp"), "-o", out, f"-L{lib}", "-ltorch", "-ltorch_cpu", "-ltorch_python",
+            "-lc10", "-lc10_hip"]
+
+
 def build(verbose: bool = False, extra_flags: list[str] | None = None, out: str | None = None) -> str:
-    """Compile the library; returns its path. Always recompiles (it is the build check)."""
+    """Compile the library, and the binding beside it; returns the library's path. Always recompiles (it
+    is the build check)."""
+    binding = BINDING_PATH if out is None else None
     out = out or LIB_PATH
     tmp = out + ".tmp"
     objdir = os.path.join(BUILD_DIR, os.path.basename(out) + ".objs")
@@ -71,11 +90,15 @@ def build(verbose: bool = False, extra_flags: list[str] | None = None, out: str 
     objs = [os.path.join(objdir, os.path.basename(src) + ".o") for src in SOURCES]
     jobs = [[hipcc(), *flags, "-c", src, "-o", obj] for src, obj in zip(SOURCES, objs)]
     workers = max(1, min(len(jobs), int(os.environ.get("MAX_JOBS", "0") or 0) or (os.cpu_count() or 1)))
+    if binding is not None:
+        jobs.insert(0, binding_command(binding + ".tmp"))
     with ThreadPoolExecutor(max_workers=workers) as pool:
         for f in [pool.submit(_run, cmd, verbose) for cmd in jobs]:
             f.result()
     _run([hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp], verbose)
     os.replace(tmp, out)
+    if binding is not None:
+        os.replace(binding + ".tmp", binding)
     return out
 
 

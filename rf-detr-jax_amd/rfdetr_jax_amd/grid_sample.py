@@ -113,6 +113,9 @@ def bilinear_grid_sample(inputs, grid, padding_mode: str = "zeros"):
         raise ValueError(f"padding_mode must be 'zeros' or 'border', got {padding_mode!r}")
     if grid.dim() != 4:
         raise ValueError(f"grid must be [N, Hg, Wg, 2], got {tuple(grid.shape)}")
+    out = _native.binding().grid_sample(inputs, grid, _native.GRID_COORDS, _native.PADDING[padding_mode], _native.SAMPLE_BILINEAR)
+    if out is not None:
+        return out
     _check(inputs, grid)
     n, gh, gw, _ = grid.shape
     out = _GridSampleFunction.apply(inputs, grid.reshape(n, gh * gw, 2), _native.GRID_COORDS, _native.PADDING[padding_mode],
@@ -136,10 +139,13 @@ def point_sample(inputs, point_coords, mode: str = "bilinear"):
     """
     if mode not in ("bilinear", "nearest"):
         raise ValueError(f"point_sample supports bilinear and nearest sampling, got {mode!r}")
+    sample = _native.SAMPLE_NEAREST if mode == "nearest" else _native.SAMPLE_BILINEAR
+    out = _native.binding().grid_sample(inputs, point_coords, _native.GRID_UNIT_POINTS, _native.PADDING["border"], sample)
+    if out is not None:
+        return out
     _check(inputs, point_coords)
     squeeze = point_coords.dim() == 3
     n = point_coords.shape[0]
     flat = point_coords.reshape(n, -1, 2)
-    sample = _native.SAMPLE_NEAREST if mode == "nearest" else _native.SAMPLE_BILINEAR
     out = _GridSampleFunction.apply(inputs, flat, _native.GRID_UNIT_POINTS, _native.PADDING["border"], sample)
     return out if squeeze else out.reshape(n, inputs.shape[1], *point_coords.shape[1:3])

@@ -17,9 +17,11 @@ Mirrors ``rfdetr_jax.models.ops`` (src/rfdetr_jax/models/ops.py):
   attention_weights)`` signature of the upstream Deformable-DETR op; ``level_start_index`` is
   checked against the prefix sums of ``spatial_shapes`` (ops.py:265-267 derives them).
 
-Differentiation is a ``torch.autograd.Function`` whose forward and backward each enqueue one
-kernel through the C ABI — the counterpart of the reference's ``jax.custom_vjp`` around its fused
-sampler (deform_pallas.py:132-178). Tensors must be on a GPU: there is no CPU path.
+Differentiation is an autograd function whose forward and backward each make one call of the C ABI —
+the counterpart of the reference's ``jax.custom_vjp`` around its fused sampler
+(deform_pallas.py:132-178): in C++ (csrc/torch_binding.cpp) for ordinary calls, in Python for what
+needs a conversion, a check's message, or torch features the C++ one passes by. Tensors must be on a
+GPU: there is no CPU path.
 """
 
 from __future__ import annotations
@@ -247,7 +249,10 @@ def ms_deform_attn_core_rows(value, spatial_shapes, sampling_locations, attentio
     Raises:
         ValueError: unknown ``sampler`` or inconsistent shapes.
     """
-    _sampler_code(sampler)
+    code = _sampler_code(sampler)
+    out = _native.binding().core(value, spatial_shapes, sampling_locations, attention_weights, code)
+    if out is not None:
+        return out
     shapes = _as_shapes(spatial_shapes)
     return _MSDeformAttnFunction.apply(value, sampling_locations, attention_weights, shapes, sampler)
 
@@ -411,5 +416,8 @@ def ms_deform_attn_fused(value, spatial_shapes, reference_points, sampling_offse
         ValueError: a ``reference_points`` trailing dimension other than 2 or 4 (as ops.py:400),
             or inconsistent shapes.
     """
+    out = _native.binding().fused(value, spatial_shapes, reference_points, sampling_offsets, attention_logits)
+    if out is not None:
+        return out
     shapes = _as_shapes(spatial_shapes)
     return _MSDeformAttnFusedFunction.apply(value, reference_points, sampling_offsets, attention_logits, shapes)

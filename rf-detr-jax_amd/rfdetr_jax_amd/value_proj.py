@@ -123,6 +123,10 @@ def value_proj_rows(x, weight, bias, n_heads, padding_mask=None):
         n_heads: number of heads.
         padding_mask: ``[B, S]`` bool, ``True`` on padded positions, or ``None``.
     """
+    if type(n_heads) is int:
+        out = _native.binding().value_proj(x, weight, bias, n_heads, padding_mask)
+        if out is not None:
+            return out
     return _ValueProjFunction.apply(x, weight, bias, n_heads, padding_mask)
 
 
