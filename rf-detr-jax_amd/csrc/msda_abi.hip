@@ -503,6 +503,28 @@ int plan_band(const Shape& s, int vbytes, int ch, const DevInfo& dev, BandPlan* 
         ++bp->bands[best];
         ++nb_total;
       }
+      // One item must not outlast the rest: while the level with the most points per band has an item
+      // longer than a CU's share of all items, it gets one more band. In points: an item costs the
+      // points of rows + 1 of its level's h rows, and 5.5 us, which is 300 points of 32 channels
+      // (18 ns each). f32, 8 heads of 32, 900 queries x 4 points: eight images of 30x40 + 15x20
+      // levels, the coarse one a single item: backward 80 us without this rule and 71 with it; two
+      // images of 64x85, 32x43, 16x22, 8x11: 79 and 76; eight of them, with items to spare, are as before.
+      const double fixed = 300.0 * 32 / s.dim, all = static_cast<double>(s.queries) * s.points;
+      auto cost = [&](int l) {
+        const int rows = (s.h[l] + bp->bands[l] - 1) / bp->bands[l];
+        return fixed + all * std::min(rows + 1, s.h[l]) / s.h[l];
+      };
+      for (;;) {
+        int top = 0;
+        double sum = 0.0;
+        for (int l = 0; l < s.levels; ++l) {
+          sum += cost(l) * bp->bands[l];
+          if (cost(l) > cost(top)) top = l;
+        }
+        const double longest = cost(top);
+        if (bp->bands[top] >= s.h[top] || longest * static_cast<double>(target) <= static_cast<double>(N) * sum) break;
+        ++bp->bands[top];
+      }
     }
   }
   bp->qblock = std::max(1, (s.queries + bp->nqb - 1) / bp->nqb);
@@ -594,8 +616,19 @@ int bwd_band_impl(const Shape& s, int ch, const void* value, int value_dtype, co
                       : 0;
   p.lds_list = bp.layout.list;
   p.lds_cnt = bp.layout.cnt;
+  // Items by falling points per band (of a level of h rows, rows + 1 of them meet a band): a level
+  // that is one item takes all of its points, and last in line such workgroups ran alone (four
+  // levels of a 64 x 85 image, 8 heads of 32, 900 queries x 4 points: 176 items of an image on 32 CUs,
+  // the last 16 of them 70 us each; with the corner reads and lane sums of the band kernel, f32 178 -> 147
+  // us for eight images, bf16 164 -> 132).
+  int order[msda::kMaxLevels];
+  for (int l = 0; l < s.levels; ++l) order[l] = l;
+  std::stable_sort(order, order + s.levels, [&](int a, int b) {
+    return static_cast<int64_t>(std::min(bp.rows[a] + 1, s.h[a])) * s.h[b] > static_cast<int64_t>(std::min(bp.rows[b] + 1, s.h[b])) * s.h[a];
+  });
   int first = 0;
-  for (int l = 0; l < s.levels; ++l) {
+  for (int i = 0; i < s.levels; ++i) {
+    const int l = order[i];
     p.lv[l] = level_desc(s, l, 0, bp.rows[l], first);
     first += bp.bands[l];
   }

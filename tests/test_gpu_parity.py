@@ -285,6 +285,27 @@ def test_kernel_variants(tune, variant, shapes):
     assert_close(ga, ra, 1e-4, "grad_attn")
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("batch,heads,dim,queries,shapes,points", [
+    (8, 8, 32, 300, ((30, 40), (15, 20)), 4),                   # the coarse level gets a second band
+    (1, 2, 32, 301, ((8, 11), (16, 22), (64, 85), (32, 43)), 3),  # coarse levels first, mostly one row per band
+    (2, 16, 16, 77, ((1, 9), (50, 61), (7, 1)), 2),             # one-row and one-column levels beside a banded one
+    (1, 3, 64, 65, ((5, 3), (48, 40), (2, 2)), 1),              # eight lanes per sample, one point
+])
+def test_band_order_over_levels(batch, heads, dim, queries, shapes, points, dtype):
+    """Levels whose items are not numbered in level order (and a level with several bands between
+    levels of one) against the C oracle, with the tolerances of this file."""
+    bf16 = dtype == "bf16"
+    value, loc, attn, grad = make_inputs(321, batch, heads, dim, queries, shapes, points)
+    if bf16:
+        value = R.bf16_round(value)
+    _note(f"band order {dtype} B={batch} H={heads} D={dim} Q={queries} P={points} {shapes}")
+    _, (gv, gl, ga) = _run(value, shapes, loc, attn, grad, bf16)
+    tol = 2e-2 if bf16 else 1e-4
+    for got, want, what in zip((gv, gl, ga), cref.backward(value, shapes, loc, attn, grad), ("value", "loc", "attn")):
+        assert_close(got, want, tol, "grad_" + what)
+
+
 def test_level_larger_than_lds():
     """A 200x120 f32 level (1.5 MB per slice) plus a small one: global-gather forward, banded backward."""
     shapes = ((200, 120), (10, 12))
