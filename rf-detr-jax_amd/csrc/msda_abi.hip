@@ -970,6 +970,19 @@ int fwd_impl(const void* value, int value_dtype, const float* loc, const float* 
   return msda_host::dispatch_fwd<float>(vec_used, ns, fused, p, plan.grid, plan.threads, plan.lds, st);
 }
 
+// fn(std::integral_constant<int, lp>) for a row of lp samples, a power of two up to 32
+template <typename F>
+void launch_fused_rows(int lp, F fn) {
+  switch (lp) {
+    case 1: fn(std::integral_constant<int, 1>{}); break;
+    case 2: fn(std::integral_constant<int, 2>{}); break;
+    case 4: fn(std::integral_constant<int, 4>{}); break;
+    case 8: fn(std::integral_constant<int, 8>{}); break;
+    case 16: fn(std::integral_constant<int, 16>{}); break;
+    default: fn(std::integral_constant<int, 32>{}); break;
+  }
+}
+
 // ------------------------------------------------------------------------------------------
 // the fused-prologue backward: prologue kernel, the core's band kernel, epilogue kernel
 
@@ -1033,6 +1046,7 @@ int fused_bwd_impl(const Shape& s, int ch, const void* value, int value_dtype, c
   fp.bq_total = static_cast<int64_t>(s.batch) * s.queries;
   fp.fpoints = static_cast<float>(s.points);
   fp.inv_points = inv_points;
+  fp.inv_heads = 1.0f / static_cast<float>(s.heads);
   for (int l = 0; l < s.levels; ++l) {
     fp.fw[l] = static_cast<float>(s.w[l]);
     fp.fh[l] = static_cast<float>(s.h[l]);
@@ -1047,7 +1061,12 @@ int fused_bwd_impl(const Shape& s, int ch, const void* value, int value_dtype, c
                      ? (lp <= 8 ? 8 : lp <= 16 ? 16 : 32)
                      : 0;
   const dim3 pgrid(static_cast<unsigned>((nsamp + 255) / 256));
-  if (nb == 8)
+  // Rows of a power of two of samples: LP is a constant of the kernel. (The entry point takes at most
+  // 64 heads, the lanes of one wave in the reference-point sum.)
+  const bool run = nb != 0 && (lp & (lp - 1)) == 0;
+  if (run)
+    launch_fused_rows(lp, [&](auto n) { hipLaunchKernelGGL(msda::fused_prologue_rows_kernel<decltype(n)::value>, pgrid, dim3(256), 0, st, fp); });
+  else if (nb == 8)
     hipLaunchKernelGGL(msda::fused_prologue_samples_kernel<8>, pgrid, dim3(256), 0, st, fp);
   else if (nb == 16)
     hipLaunchKernelGGL(msda::fused_prologue_samples_kernel<16>, pgrid, dim3(256), 0, st, fp);
@@ -1072,7 +1091,11 @@ int fused_bwd_impl(const Shape& s, int ch, const void* value, int value_dtype, c
     const int G = 256 / (s.heads * lp), hp = 1 << hp_shift;
     const dim3 sgrid(static_cast<unsigned>((fp.bq_total + G - 1) / G));
     const size_t lds = static_cast<size_t>(G) * (s.heads * lp + s.levels * hp) * sizeof(float4);
-    if (nb == 8)
+    if (run)
+      launch_fused_rows(lp, [&](auto n) {
+        hipLaunchKernelGGL(msda::fused_epilogue_rows_kernel<decltype(n)::value>, sgrid, dim3(256), 0, st, fp, G, hp_shift);
+      });
+    else if (nb == 8)
       hipLaunchKernelGGL(msda::fused_epilogue_samples_kernel<8>, sgrid, dim3(256), lds, st, fp, G, hp);
     else if (nb == 16)
       hipLaunchKernelGGL(msda::fused_epilogue_samples_kernel<16>, sgrid, dim3(256), lds, st, fp, G, hp);

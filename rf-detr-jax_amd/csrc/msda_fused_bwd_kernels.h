@@ -3,8 +3,8 @@
 // msda_fused_bwd replaces the JAX autodiff VJP of MSDeformAttn.__call__ from the offsets to the
 // core call (src/rfdetr_jax/models/ops.py:388-410): locations from reference points and offsets
 // (:388-399, precise_divide :46-62), softmax weights (:403-404), the core (:408-410). It runs as
-//  1. fused_prologue_kernel: one thread per (b, q, h) row forms the row's locations and softmax
-//     weights (the same arithmetic as msda_fused_fwd's kernels: fused_location_at, softmax_stats /
+//  1. fused_prologue_kernel: one thread per (b, q, h) row (or per sample, below) forms the row's
+//     locations and softmax weights (the same arithmetic as msda_fused_fwd's kernels: fused_location_at, softmax_stats /
 //     softmax_weight) into the workspace;
 //  2. the core backward (bwd_band_kernel) on them, writing grad_value, the gradient of the
 //     locations (into grad_sampling_offsets, or the workspace) and of the weights (into
@@ -17,6 +17,8 @@
 // reference-point partials are added in head order by the part-sum kernel (with query blocks) or
 // ref_head_sum_kernel.
 #pragma once
+
+#include <utility>
 
 #include "msda_band_kernels.h"
 
@@ -35,6 +37,7 @@ struct FusedRowParams {
   int ref_dim, heads, levels, points;
   int64_t bq_total;     // B * Q
   float inv_points, fpoints;
+  float inv_heads;      // 1.0f / heads
   float fw[kMaxLevels], fh[kMaxLevels];
 };
 
@@ -115,11 +118,12 @@ __global__ void __launch_bounds__(256) fused_epilogue_kernel(const FusedRowParam
 // The same two steps with one thread per sample (b, q, h, k), for rows of at most NB samples over at
 // most four levels (every RF-DETR shape) and fewer than 2^31 samples. Each lane loads its own
 // offset, location gradient and reference point: loads and stores are contiguous runs, and there
-// are LP times as many threads to hide latency as the row kernels above have. When LP is a power of
-// two a row lies within one wave: each lane loads its own logit (and dA) and forms one exponential,
-// and the row's statistics and sums come from the other lanes by shuffles (row_stats_lanes);
-// otherwise every lane of a row loads the row's logits (one broadcast address per row) and forms
-// them all. The arithmetic and its order are those of the row kernels either way.
+// are LP times as many threads to hide latency as the row kernels above have. The *_rows kernels
+// take LP as a constant, a power of two (a row then lies within one wave): each lane loads its own
+// logit (and dA) and forms one exponential, and the row's statistics and sums come from the other
+// lanes. In the *_samples kernels, for any other LP, every lane of a row loads the row's logits (one
+// broadcast address per row) and forms them all. The arithmetic and its order are those of the row
+// kernels either way.
 __device__ __forceinline__ float level_pick(int l, const float (&a)[kMaxLevels]) {
   return l == 0 ? a[0] : l == 1 ? a[1] : l == 2 ? a[2] : a[3];
 }
@@ -136,43 +140,104 @@ __device__ __forceinline__ SoftmaxStats row_stats(const float (&x)[NB], int LP) 
   return st;
 }
 
-// The softmax statistics of a row held one logit per lane (xk), its LP lanes consecutive and
-// LP-aligned in the wave (LP a power of two dividing 64), for every lane of the row: the maximum by
-// a butterfly (exact in any order), the sum of the lanes' exp(x - m) (ek) gathered and added in
-// sample order from 0, as row_stats and softmax_stats add them, so the weights are theirs bit for
-// bit with one exponential per lane instead of LP. Every lane of the wave must take part.
-__device__ __forceinline__ SoftmaxStats row_stats_lanes(float xk, int LP, float& ek) {
-  SoftmaxStats st{xk, 0.0f};
-  for (int o = LP >> 1; o > 0; o >>= 1) st.m = fmaxf(st.m, __shfl_xor(st.m, o, LP));
-  ek = expf(xk - st.m);
-  for (int u = 0; u < LP; ++u) st.s += __shfl(ek, u, LP);
-  return st;
+// The value that lane U of each run of LP consecutive, LP-aligned lanes holds, for every lane of the
+// run. Moves between lanes cost no LDS cycles this way: quad_perm for runs of 2 and 4, row_newbcast
+// for 8 (two halves of a row of 16) and 16, readlane for 32. Every lane of the wave must take part.
+template <int LP, int U>
+__device__ __forceinline__ float run_lane(float x) {
+  const int v = __float_as_int(x);
+  if constexpr (LP == 1) return x;
+  else if constexpr (LP == 2) return __int_as_float(__builtin_amdgcn_mov_dpp(v, U * 5 + (2 + U) * 80, 0xF, 0xF, false));
+  else if constexpr (LP == 4) return __int_as_float(__builtin_amdgcn_mov_dpp(v, U * 0x55, 0xF, 0xF, false));
+  else if constexpr (LP == 8) {
+    const int lo = __builtin_amdgcn_update_dpp(v, v, 0x150 + U, 0xF, 0x3, false);
+    return __int_as_float(__builtin_amdgcn_update_dpp(lo, v, 0x158 + U, 0xF, 0xC, false));
+  } else if constexpr (LP == 16) return __int_as_float(__builtin_amdgcn_mov_dpp(v, 0x150 + U, 0xF, 0xF, false));
+  else {
+    static_assert(LP == 32, "runs of at most 32 lanes");
+    const int lo = __builtin_amdgcn_readlane(v, U), hi = __builtin_amdgcn_readlane(v, 32 + U);
+    return __int_as_float((threadIdx.x & 32) != 0 ? hi : lo);
+  }
 }
 
-__device__ __forceinline__ bool rows_in_lanes(int LP) { return (LP & (LP - 1)) == 0 && LP <= 64; }
+// f(U's value) for U = 0 .. LP - 1, in order.
+template <int LP, typename F, int... U>
+__device__ __forceinline__ void run_each(float x, F f, std::integer_sequence<int, U...>) {
+  (f(run_lane<LP, U>(x)), ...);
+}
+
+template <int LP>
+__device__ __forceinline__ float run_max(float x) {
+  auto step = [&](int moved) { x = fmaxf(x, __int_as_float(moved)); };
+  if constexpr (LP >= 2) step(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xF, 0xF, false));   // lane ^ 1
+  if constexpr (LP >= 4) step(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x4E, 0xF, 0xF, false));   // lane ^ 2
+  if constexpr (LP >= 8) step(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x141, 0xF, 0xF, false));  // the other quad of 8
+  if constexpr (LP >= 16) step(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x140, 0xF, 0xF, false)); // the other half of 16
+  if constexpr (LP == 32) x = fmaxf(run_lane<32, 0>(x), run_lane<32, 16>(x));
+  return x;
+}
+
+// The softmax weight of the logit x of each lane within its row: the maximum by a butterfly (exact in
+// any order), the sum of the lanes' exp(x - m) added in sample order from 0, as row_stats and
+// softmax_stats add them, so the weights are theirs bit for bit with one exponential per lane instead
+// of LP.
+template <int LP>
+__device__ __forceinline__ float run_softmax(float x) {
+  const float e = expf(x - run_max<LP>(x));
+  float s = 0.0f;
+  run_each<LP>(e, [&](float v) { s += v; }, std::make_integer_sequence<int, LP>{});
+  return e / s;
+}
+
+// S = fma(a_U, d_U, S) for U = 0 .. LP - 1, in order.
+template <int LP, int... U>
+__device__ __forceinline__ void run_dot(float a, float d, float& S, std::integer_sequence<int, U...>) {
+  ((S = fmaf(run_lane<LP, U>(a), run_lane<LP, U>(d), S)), ...);
+}
+
+// Level of sample k (at most four levels of `points`).
+__device__ __forceinline__ int sample_level(int k, int points) {
+  return (k >= points ? 1 : 0) + (k >= 2 * points ? 1 : 0) + (k >= 3 * points ? 1 : 0);
+}
+
+// n / d for 0 <= n < 512 and 1 <= d <= 64, inv = 1.0f / d: n + 0.5 is at least half a unit of 1 / d
+// from a multiple of d, and the product's error is far below that.
+__device__ __forceinline__ int small_div(int n, float inv) { return static_cast<int>((static_cast<float>(n) + 0.5f) * inv); }
+
+// These two kernels are bound by their vector instructions, not by memory: with runtime LP, shuffles
+// through the LDS crossbar and integer divisions per lane, 921600 samples (8 x 900 x 8 heads x 16,
+// 22 MB in and out) took 11.1 us forward and, 30 MB, 18.2 us back; now 7.2 and 11.0. For rows of a
+// power of two up to 32 samples, four levels and the entry point's 64 heads.
+template <int LP>
+__global__ void __launch_bounds__(256) fused_prologue_rows_kernel(const FusedRowParams p) {
+  const int t = threadIdx.x, k = t & (LP - 1);
+  const uint32_t row0 = blockIdx.x * (256u / LP), bq0 = row0 / static_cast<uint32_t>(p.heads);  // uniform
+  const uint32_t row = row0 + static_cast<uint32_t>(t / LP);
+  const bool on = row < static_cast<uint32_t>(p.bq_total) * static_cast<uint32_t>(p.heads);
+  const uint32_t idx = row * LP + static_cast<uint32_t>(k);
+  const int l = sample_level(k, p.points);
+  float x = 0.0f;
+  float2 o = make_float2(0.0f, 0.0f);
+  float4 r = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (on) {
+    x = p.logits[idx];
+    o = reinterpret_cast<const float2*>(p.off)[idx];
+    const int rem = static_cast<int>(row - bq0 * static_cast<uint32_t>(p.heads));  // < heads + 256
+    r = fused_row_ref(p, bq0 + static_cast<uint32_t>(small_div(rem, p.inv_heads)), l);
+  }
+  const float a = run_softmax<LP>(x);
+  if (!on) return;
+  float2 tt;
+  reinterpret_cast<float2*>(p.loc)[idx] =
+      fused_location_at(o, r, tt, level_pick(l, p.fw), level_pick(l, p.fh), p.ref_dim, p.inv_points, p.fpoints);
+  p.attn[idx] = a;
+}
 
 template <int NB>
 __global__ void __launch_bounds__(256) fused_prologue_samples_kernel(const FusedRowParams p) {
   const uint32_t LP = static_cast<uint32_t>(p.levels * p.points);
   const uint32_t total = static_cast<uint32_t>(p.bq_total * p.heads) * LP;
-  uint32_t idx = blockIdx.x * 256u + threadIdx.x;  // (b, q, h, k)
-  if (rows_in_lanes(static_cast<int>(LP))) {  // uniform: one exponential per lane, the row's sums by shuffles
-    const bool on = idx < total;
-    if (!on) idx = 0;  // whole rows only, so the lanes past the end form rows of their own
-    const uint32_t row = idx / LP, k = idx - row * LP;
-    const int l = static_cast<int>(k) / p.points;
-    const float xk = p.logits[idx];
-    float ek;
-    const SoftmaxStats st = row_stats_lanes(xk, static_cast<int>(LP), ek);
-    if (!on) return;
-    const float2 o = reinterpret_cast<const float2*>(p.off)[idx];
-    const float4 r = fused_row_ref(p, row / static_cast<uint32_t>(p.heads), l);
-    float2 t;
-    reinterpret_cast<float2*>(p.loc)[idx] =
-        fused_location_at(o, r, t, level_pick(l, p.fw), level_pick(l, p.fh), p.ref_dim, p.inv_points, p.fpoints);
-    p.attn[idx] = ek / st.s;  // softmax_weight(xk, st)
-    return;
-  }
+  const uint32_t idx = blockIdx.x * 256u + threadIdx.x;  // (b, q, h, k)
   if (idx >= total) return;
   const uint32_t row = idx / LP, k = idx - row * LP;
   const int l = static_cast<int>(k) / p.points;
@@ -210,16 +275,12 @@ __global__ void __launch_bounds__(256) fused_epilogue_samples_kernel(const Fused
   const uint32_t row = bq * static_cast<uint32_t>(H) + static_cast<uint32_t>(h);
   const uint32_t idx = row * static_cast<uint32_t>(LP) + static_cast<uint32_t>(k);
   const bool want_dl = p.dlogits != nullptr, want_loc = p.dloc != nullptr;  // uniform
-  const bool lanes = rows_in_lanes(LP);  // uniform: each lane loads its own logit and dA only
   float x[NB], d[NB];
   float xk = 0.0f, dk = 0.0f;
   float2 gl = make_float2(0.0f, 0.0f), o = make_float2(0.0f, 0.0f);
   float4 ref = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   if (on) {
-    if (want_dl && lanes) {
-      xk = p.logits[idx];
-      dk = p.dlogits[idx];
-    } else if (want_dl) {
+    if (want_dl) {
       const float* __restrict__ lg = p.logits + static_cast<size_t>(row) * LP;
       const float* __restrict__ dl = p.dlogits + static_cast<size_t>(row) * LP;
 #pragma unroll
@@ -240,14 +301,7 @@ __global__ void __launch_bounds__(256) fused_epilogue_samples_kernel(const Fused
   }
   wait_vmem();
   __syncthreads();  // the rows' dA are read before any of them is overwritten
-  if (want_dl && lanes) {  // every lane of the block takes part in the row shuffles
-    float ek;
-    const SoftmaxStats st = row_stats_lanes(xk, LP, ek);
-    const float wk = ek / st.s;  // softmax_weight(xk, st)
-    float S = 0.0f;
-    for (int u = 0; u < LP; ++u) S = fmaf(__shfl(wk, u, LP), __shfl(dk, u, LP), S);  // as the row kernel, in order
-    if (on) p.dlogits[idx] = wk * (dk - S);
-  } else if (on && want_dl) {
+  if (on && want_dl) {
     const SoftmaxStats st = row_stats<NB>(x, LP);
     float S = 0.0f;
 #pragma unroll
@@ -304,6 +358,73 @@ __global__ void __launch_bounds__(256) fused_epilogue_samples_kernel(const Fused
       dd[2] = v[0].z;
       dd[3] = v[0].w;
     }
+  }
+}
+
+// Constant LP: G whole (b, q) groups per workgroup (256 / (heads * LP) >= 1). A lane reads and writes
+// only its own sample's logit, dA and location gradient, so the in-place step needs no barrier. The
+// reference-point shares go through LDS, one array per component (rows a word apart in their banks),
+// then each lane of (group, level, component, head) adds its level's points in order, and the heads
+// are the lanes of a butterfly, the pairwise tree of the row kernel. hp = 2^hp_shift >= heads, <= 64.
+constexpr int kEpiPlane = 256 + 256 + 2;  // words of one component: 256 samples, one word of skew per row
+template <int LP>
+__global__ void __launch_bounds__(256) fused_epilogue_rows_kernel(const FusedRowParams p, int G, int hp_shift) {
+  __shared__ float cbuf[4 * kEpiPlane];
+  const int H = p.heads, L = p.levels, P = p.points;
+  const int t = threadIdx.x, k = t & (LP - 1), rl = t / LP;
+  const int g = small_div(rl, p.inv_heads), l = sample_level(k, P);
+  const uint32_t bq0 = blockIdx.x * static_cast<uint32_t>(G), bq = bq0 + static_cast<uint32_t>(g);
+  const bool on = g < G && bq < static_cast<uint32_t>(p.bq_total);
+  const uint32_t idx = (bq0 * static_cast<uint32_t>(H) + static_cast<uint32_t>(rl)) * LP + static_cast<uint32_t>(k);
+  const bool want_dl = p.dlogits != nullptr, want_loc = p.dloc != nullptr;  // uniform
+  float x = 0.0f, d = 0.0f;
+  float2 gl = make_float2(0.0f, 0.0f), o = make_float2(0.0f, 0.0f);
+  float4 ref = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (on) {
+    if (want_dl) {
+      x = p.logits[idx];
+      d = p.dlogits[idx];
+    }
+    if (want_loc) {
+      gl = reinterpret_cast<const float2*>(p.dloc)[idx];
+      o = reinterpret_cast<const float2*>(p.off)[idx];
+      ref = fused_row_ref(p, bq, l);
+    }
+  }
+  if (want_dl) {  // every lane of the block takes part
+    const float a = run_softmax<LP>(x);
+    // sum of a_j dA_j, in sample order, one rounding per term as the row kernel's fmaf: both factors
+    // are moved, not their product
+    float S = 0.0f;
+    run_dot<LP>(a, d, S, std::make_integer_sequence<int, LP>{});
+    if (on) p.dlogits[idx] = a * (d - S);
+  }
+  if (!want_loc) return;  // uniform
+  float r4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (on) {
+    const float fw = level_pick(l, p.fw), fh = level_pick(l, p.fh);
+    float2 tt;
+    fused_location_at(o, ref, tt, fw, fh, p.ref_dim, p.inv_points, p.fpoints);
+    const float2 go = fused_offset_grad(gl, ref, tt, fw, fh, p.ref_dim, p.inv_points, p.fpoints, r4);
+    if (p.doff != nullptr) reinterpret_cast<float2*>(p.doff)[idx] = go;
+  }
+  if (p.dref == nullptr) return;  // uniform
+#pragma unroll
+  for (int c = 0; c < 4; ++c) cbuf[c * kEpiPlane + t + rl] = r4[c];
+  __syncthreads();
+  const int hp = 1 << hp_shift, total = (G * L * 4) << hp_shift;
+  for (int i0 = 0; i0 < total; i0 += 256) {  // uniform: every lane takes part in the shuffles
+    const int i = i0 + t, h2 = i & (hp - 1), c = (i >> hp_shift) & 3, gl2 = (i >> hp_shift) >> 2;
+    const int g2 = gl2 / L, l2 = gl2 - g2 * L;
+    float v = 0.0f;
+    if (i < total && h2 < H) {
+      const int r2 = g2 * H + h2;
+      const float* s = cbuf + c * kEpiPlane + r2 * (LP + 1) + l2 * P;
+      for (int pt = 0; pt < P; ++pt) v += s[pt];
+    }
+    v = sum_lanes(v, hp);
+    if (i < total && h2 == 0 && c < p.ref_dim && bq0 + static_cast<uint32_t>(g2) < static_cast<uint32_t>(p.bq_total))
+      p.dref[(static_cast<size_t>(bq0) * L + static_cast<size_t>(gl2)) * p.ref_dim + c] = v;
   }
 }
 

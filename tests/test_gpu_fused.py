@@ -228,6 +228,31 @@ def test_fused_row_kernels(tune, case, ref_dim):
     _check(out, grads, want_out, want_grads, False)
 
 
+@pytest.mark.parametrize("needs", [(True, True, True, True), (False, True, False, False), (False, False, False, True)],
+                         ids=["all", "ref", "logits"])
+@pytest.mark.parametrize("heads,queries,shapes,points", [
+    (3, 43, ((64, 96),), 1),                              # one sample per row, on a banded level
+    (5, 41, ((64, 96), (2, 3)), 1),                       # 2, heads that do not fill the workgroup
+    (64, 3, ((9, 7), (4, 4), (2, 3), (1, 1)), 1),         # 4, one group of 64 heads fills it
+    (7, 37, ((9, 7), (4, 4), (2, 3), (1, 1)), 2),         # 8
+    (3, 21, ((9, 7), (4, 4)), 8),                         # 16, eight points per level
+    (7, 5, ((9, 7), (4, 4), (2, 3), (1, 1)), 8),          # 32, one group of 224 threads
+])
+def test_fused_rows_of_constant_length(tune, heads, queries, shapes, points, needs):
+    """Rows of 1 to 32 samples (a power of two) and ragged last workgroups: bit for bit what the
+    kernels with one thread per row give, a wholly masked row's NaN included."""
+    _note(f"fused constant rows H={heads} Q={queries} P={points} {shapes} {needs}")
+    value, ref, off, logits, grad = make_fused_inputs(16, 1, heads, 16, queries, shapes, points, 4)
+    logits[:, 1, -1] = -np.inf
+    logits[:, ::4, :, -1] = -np.inf
+    _, grads = _run_fused(value, shapes, ref, off, logits, grad, needs=needs)
+    tune({"MSDA_FUSED_PER_SAMPLE": "0"})
+    _, grads0 = _run_fused(value, shapes, ref, off, logits, grad, needs=needs)
+    for name, g, g0 in zip(("grad_reference_points", "grad_sampling_offsets", "grad_attention_logits"), grads[1:], grads0[1:]):
+        assert (g is None) == (g0 is None), name
+        assert g is None or np.array_equal(g, g0, equal_nan=True), name
+
+
 def test_fused_three_points_four_heads():
     """Four heads, three points (n_points not a power of two: the box form divides), one small
     level; the epilogue sums grad_reference_points over four head lanes."""
