@@ -76,7 +76,8 @@ int msda_grid_sample_fwd(const void* input, int dtype, const float* grid, int gr
   if ((rc = msda_host::device_attrs(&lds_bytes, &cus)) != MSDA_OK) return rc;
   // Staged when one plane fits in a third of the LDS (three workgroups per CU) and there are enough
   // points per plane to pay for the copy (measured on MI355X, 400 one-channel 112x112 f32 planes:
-  // 2352 points 9.4 us staged against 21 us gathered through L2; 784 points 9.4 against 8.2).
+  // 2352 points 7.5 us staged against 9.8 gathered through L2, 784 points 4.8 gathered; bf16 planes,
+  // 2352 points 7.3 against 12.5).
   const int budget = std::min(lds_bytes / 3, 64 * 1024);
   const int64_t plane_bytes = static_cast<int64_t>(height) * width * static_cast<int64_t>(eb);
   if (plane_bytes <= budget && static_cast<int64_t>(n_points) * 12 >= static_cast<int64_t>(height) * width &&
@@ -127,32 +128,36 @@ int msda_grid_sample_bwd(const void* input, int dtype, const float* grid, int gr
   msda::GridSampleParams p = gs_params(input, dtype, grid, grid_kind, n, channels, height, width, n_points, padding_mode, sample_mode);
   p.gout = grad_output;
   if (grad_input != nullptr) {
-    // the accumulator of one workgroup: a chunk of channels x a band of rows, within 64 KB so
-    // that several workgroups share a CU; whole planes when they fit
+    // the f64 accumulator of one workgroup: a chunk of channels x a band of rows, within 64 KB so that
+    // workgroups share a CU (one row past that up to 128 KB); whole planes when they fit
     const int budget = std::min(lds_bytes, 64 * 1024);
-    const int64_t row_bytes = static_cast<int64_t>(width) * 4;
-    if (row_bytes > budget) return fail(MSDA_ERR_UNSUPPORTED, "width %d exceeds the grad_input accumulator (%d bytes of LDS)", width, budget);
+    const int64_t row_bytes = static_cast<int64_t>(width) * 8;
+    if (row_bytes > std::min(lds_bytes, 128 * 1024))
+      return fail(MSDA_ERR_UNSUPPORTED, "width %d exceeds the grad_input accumulator (%d bytes of LDS)", width, lds_bytes);
     const int64_t plane_bytes = row_bytes * height;
     if (plane_bytes <= budget) {
       p.band_rows = height;
       p.chunk = static_cast<int>(std::min<int64_t>(channels, budget / plane_bytes));
     } else {
       p.chunk = 1;
-      p.band_rows = static_cast<int>(budget / row_bytes);
+      p.band_rows = static_cast<int>(std::max<int64_t>(1, budget / row_bytes));
     }
-    // at least four workgroups per CU (measured on MI355X with 400 one-channel 112x112 masks: 400
-    // whole-plane workgroups leave CUs idle); each band re-reads the slice's points, which are few
-    const int64_t chunks = (channels + p.chunk - 1) / p.chunk;
-    const int64_t want_bands = (4 * static_cast<int64_t>(cus) + n * chunks - 1) / std::max<int64_t>(1, n * chunks);
+    // Four workgroups of 512 per CU: 400 one-channel 112x112 f32 planes, 784 and 2352 points, 10.9
+    // and 14.3 us (two: 11.2 and 15.1; four of 256: 10.8 and 17.6). Every band scans the slice's
+    // points, so past one workgroup per CU at most 8 bands: 40 planes in 26 bands 7.0 us, in 8 bands 5.1.
+    const int64_t units = static_cast<int64_t>(n) * ((channels + p.chunk - 1) / p.chunk);
+    const int64_t fill = (static_cast<int64_t>(cus) + units - 1) / units;
+    const int64_t want_bands = std::min((4 * static_cast<int64_t>(cus) + units - 1) / units, std::max<int64_t>(8, fill));
     const int64_t bands_now = (height + p.band_rows - 1) / p.band_rows;
     if (want_bands > bands_now) p.band_rows = static_cast<int>(std::max<int64_t>(1, (height + want_bands - 1) / want_bands));
     const int64_t groups = static_cast<int64_t>(n) * ((channels + p.chunk - 1) / p.chunk) * ((height + p.band_rows - 1) / p.band_rows);
     if (groups > 0x7fffffff) return fail(MSDA_ERR_UNSUPPORTED, "grad_input grid too large");
     p.ginput = grad_input;
+    p.bwd_vec = dtype == MSDA_DTYPE_F32 && width % 4 == 0 && aligned_to(grad_input, 16);
     const int lds = static_cast<int>(static_cast<int64_t>(p.chunk) * p.band_rows * row_bytes);
     static std::atomic<int> granted[msda_host::kMaxDevices];
     if ((rc = msda_host::allow_lds(msda::gs_bwd_input_kernel, lds, granted)) != MSDA_OK) return rc;
-    hipLaunchKernelGGL(msda::gs_bwd_input_kernel, dim3(static_cast<unsigned>(groups)), dim3(256), lds, st, p);
+    hipLaunchKernelGGL(msda::gs_bwd_input_kernel, dim3(static_cast<unsigned>(groups)), dim3(512), lds, st, p);
     if ((rc = msda_host::check_launch("grid sample backward (input)")) != MSDA_OK) return rc;
   }
   if (grad_grid != nullptr && n_points > 0) {

@@ -11,9 +11,9 @@
 //    and samples every point from there; out[n, c, p] is written by consecutive lanes.
 //  * gs_fwd_kernel — otherwise: one lane per (slice n, point p), the point's corners and weights
 //    once, then every channel's four corner values gathered through L2.
-//  * gs_bwd_input_kernel — one workgroup per (slice, chunk of channels, band of rows): an f32
+//  * gs_bwd_input_kernel — one workgroup per (slice, chunk of channels, band of rows): an f64
 //    accumulator for the band's pixels of those channels in LDS, every point of the slice scattered
-//    into it (LDS float atomics), then the band written once in the input dtype. grad_input needs
+//    into it (LDS atomics), then the band written once in the input dtype. grad_input needs
 //    no zero-fill and no global atomics; each element has one writer.
 //  * gs_bwd_grid_kernel — one lane per point: the gradient of the sample position, summed over
 //    channels (bilinear only; nearest sampling has none).
@@ -24,7 +24,7 @@
 #include <cstdint>
 #include <type_traits>
 
-#include "msda_kernels.h"  // stage_copy, bf16_to_f32, MSDA_LDS
+#include "msda_kernels.h"  // stage_copy, xcd_logical, bf16_to_f32, MSDA_LDS
 
 namespace msda {
 
@@ -41,6 +41,7 @@ struct GridSampleParams {
   int border;             // padding_mode "border" (else "zeros")
   int nearest;            // nearest sampling (border padding; segmentation.py:173-186)
   int chunk, band_rows;   // gs_bwd_input_kernel: channels and image rows per workgroup
+  int bwd_vec;            // gs_bwd_input_kernel: f32, rows of whole quads, grad_input 16-byte aligned
   int fwd_chunk;          // gs_fwd_lds_kernel: channel planes staged per workgroup
   int fwd_split;          // gs_fwd_lds_kernel: workgroups sharing one (slice, chunk)'s points
   int fwd_vec16;          // gs_fwd_lds_kernel: the staged planes may be copied 16 bytes at a time
@@ -129,12 +130,16 @@ __device__ __forceinline__ GsCorners gs_corners(float gx, float gy, const GridSa
   return k;
 }
 
-// One lane per (slice, point); n * points < 2^31 (checked on the host), so indices are 32-bit.
+// One lane per (slice, point); n * points < 2^31 (checked on the host), so indices are 32-bit. The
+// workgroups of a slice run on one XCD, so its planes are read into one L2 (in hardware order every
+// XCD with a workgroup of the slice reads the same cache lines): 400 one-channel 112x112 f32 planes,
+// 784 points each, 9.5 -> 4.8 us (nearest 4.9 -> 3.5).
 __global__ void __launch_bounds__(256) gs_fwd_kernel(const GridSampleParams p) {
   const uint32_t total = static_cast<uint32_t>(p.n) * static_cast<uint32_t>(p.points);
   const int64_t plane = static_cast<int64_t>(p.h) * p.w;
   const bool bf = p.bf16 != 0;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
+  const uint32_t block = static_cast<uint32_t>(xcd_logical(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x)));
+  for (uint32_t i = block * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
     const uint32_t n32 = i / static_cast<uint32_t>(p.points);
     const int64_t n = n32;
     const int pt = static_cast<int>(i - n32 * static_cast<uint32_t>(p.points));
@@ -155,17 +160,22 @@ __global__ void __launch_bounds__(256) gs_fwd_kernel(const GridSampleParams p) {
   }
 }
 
+// Points of one lane whose grid entries are requested before the staging copy or the zero-fill.
+constexpr int kGsAhead = 4;
+
 // Staged forward: workgroup = (slice n, chunk of channels, share of the points). The chunk's
 // planes (consecutive in [N, C, H, W]) are copied into LDS once in the input dtype (stage_copy:
 // global_load_lds_dwordx4 when rows allow 16-byte copies), then each lane samples its points from
 // LDS: the corner gathers of a wave touch random words, which from L2 would cost a cache line each.
-// The workgroups of one slice are consecutive ids, so they run on one XCD and share its L2.
+// Bound by the latency of its two reads, so the lane's first points are requested before the copy;
+// the workgroups of one slice are consecutive logical ids (xcd_logical), which share an L2.
+// 400 one-channel 112x112 f32 planes, 2352 points each: 11.8 -> 7.5 us.
 template <typename VT>
 __global__ void __launch_bounds__(512) gs_fwd_lds_kernel(const GridSampleParams p) {
   extern __shared__ __align__(16) unsigned char gs_raw[];
   VT* plane_lds = reinterpret_cast<VT*>(gs_raw);
   const int nchunks = (p.c + p.fwd_chunk - 1) / p.fwd_chunk;
-  int id = blockIdx.x;
+  int id = xcd_logical(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
   const int share = id % p.fwd_split;
   id /= p.fwd_split;
   const int chunk = id % nchunks;
@@ -174,18 +184,23 @@ __global__ void __launch_bounds__(512) gs_fwd_lds_kernel(const GridSampleParams 
   const int plane = p.h * p.w;
   const bool bf = p.bf16 != 0;
   const VT* src = static_cast<const VT*>(p.input) + (static_cast<int64_t>(n) * p.c + c0) * plane;
-  stage_copy<VT>(plane_lds, src, (c1 - c0) * plane, p.fwd_vec16 != 0);
-  __syncthreads();
   const int per = (p.points + p.fwd_split - 1) / p.fwd_split;
   const int pt0 = share * per, pt1 = min(p.points, pt0 + per);
   const float2* grid = reinterpret_cast<const float2*>(p.grid) + static_cast<int64_t>(n) * p.points;
+  // the lane's points are first + o, o = 0, step, 2 step .. < left (unsigned: no overflow at any count)
+  const int first = pt0 + static_cast<int>(threadIdx.x);
+  const uint32_t left = first < pt1 ? static_cast<uint32_t>(pt1 - first) : 0u, step = blockDim.x;
+  float2 ahead[kGsAhead];
+#pragma unroll
+  for (int u = 0; u < kGsAhead; ++u) ahead[u] = u * step < left ? grid[first + u * step] : make_float2(0.0f, 0.0f);
+  stage_copy<VT>(plane_lds, src, (c1 - c0) * plane, p.fwd_vec16 != 0);
+  __syncthreads();
   const MSDA_LDS VT* pl_all = (const MSDA_LDS VT*)(plane_lds);
   auto rd = [&](const MSDA_LDS VT* pl, int i) -> float {
     if constexpr (std::is_same<VT, float>::value) return pl[i];
     else return bf16_to_f32(pl[i]);
   };
-  for (int pt = pt0 + threadIdx.x; pt < pt1; pt += blockDim.x) {
-    const float2 g = grid[pt];
+  auto sample = [&](uint32_t pt, float2 g) {
     const GsCorners k = gs_corners(g.x, g.y, p);
     for (int c = c0; c < c1; ++c) {
       const MSDA_LDS VT* pl = pl_all + (c - c0) * plane;
@@ -197,15 +212,26 @@ __global__ void __launch_bounds__(512) gs_fwd_lds_kernel(const GridSampleParams 
       }
       gs_store(p.out, (static_cast<int64_t>(n) * p.c + c) * p.points + pt, v, bf);
     }
-  }
+  };
+#pragma unroll
+  for (int u = 0; u < kGsAhead; ++u)
+    if (u * step < left) sample(first + u * step, ahead[u]);
+  for (uint32_t o = kGsAhead * step; o < left; o += step) sample(first + o, grid[first + o]);
 }
 
-// Workgroup = (slice n, channel chunk, row band); LDS: chunk x band_rows x W floats.
-__global__ void __launch_bounds__(256) gs_bwd_input_kernel(const GridSampleParams p) {
-  extern __shared__ __align__(16) float gs_acc[];
+// Workgroup = (slice n, channel chunk, row band); LDS: chunk x band_rows x W doubles. The sums are f64:
+// an f32 LDS add of a wave took about 60 cycles here, an f64 add a third of that (400 one-channel
+// 112x112 f32 planes, 2352 points each: 26.1 us with f32 sums, 17.6 with f64), and the result is the
+// f64 sum rounded once. The bands of a slice, which read the same points, are consecutive logical ids
+// (xcd_logical). A lane's first points and their gradients are requested before the zero-fill, and a
+// row of whole f32 quads is written 16 bytes at a time (`vec`). From f32 sums without these, at 784
+// points 17.5 -> 10.9 us (writing the planes takes 4), at 2352 31.0 -> 14.2; 8 x 256 channels of 40x40,
+// 900 points: 54.9 -> 15.4.
+__global__ void __launch_bounds__(512) gs_bwd_input_kernel(const GridSampleParams p) {
+  extern __shared__ __align__(16) double gs_acc[];
   const int nchunks = (p.c + p.chunk - 1) / p.chunk;
   const int nbands = (p.h + p.band_rows - 1) / p.band_rows;
-  int id = blockIdx.x;
+  int id = xcd_logical(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
   const int band = id % nbands;
   id /= nbands;
   const int chunk = id % nchunks;
@@ -215,18 +241,33 @@ __global__ void __launch_bounds__(256) gs_bwd_input_kernel(const GridSampleParam
   const int w = p.w;
   const int band_px = (r1 - r0) * w;
   const int cells = (c1 - c0) * band_px;
-  for (int i = threadIdx.x; i < cells; i += blockDim.x) gs_acc[i] = 0.0f;
+  const bool bf = p.bf16 != 0, vec = p.bwd_vec != 0;
+  const float2* grid = reinterpret_cast<const float2*>(p.grid) + static_cast<int64_t>(n) * p.points;
+  const int64_t go0 = (static_cast<int64_t>(n) * p.c + c0) * p.points;  // the chunk's first grad_output row
+  const int first = static_cast<int>(threadIdx.x);  // the lane's points, as in gs_fwd_lds_kernel
+  const uint32_t left = first < p.points ? static_cast<uint32_t>(p.points - first) : 0u, step = blockDim.x;
+  float2 ahead[kGsAhead];
+  float go_ahead[kGsAhead];
+#pragma unroll
+  for (int u = 0; u < kGsAhead; ++u) {
+    const bool in = u * step < left;
+    ahead[u] = in ? grid[first + u * step] : make_float2(0.0f, 0.0f);
+    go_ahead[u] = in ? gs_load(p.gout, go0 + first + u * step, bf) : 0.0f;
+  }
+  if (vec) {
+    for (int i = threadIdx.x; i < cells / 2; i += blockDim.x) reinterpret_cast<double2*>(gs_acc)[i] = make_double2(0.0, 0.0);
+  } else {
+    for (int i = threadIdx.x; i < cells; i += blockDim.x) gs_acc[i] = 0.0;
+  }
   __syncthreads();
-  const bool bf = p.bf16 != 0;
   const int lo = r0 * w, hi = r1 * w;  // the band's flat pixel range in the plane
-  for (int pt = threadIdx.x; pt < p.points; pt += blockDim.x) {
-    const float2 g = reinterpret_cast<const float2*>(p.grid)[static_cast<int64_t>(n) * p.points + pt];
+  auto scatter = [&](uint32_t pt, float2 g, float go_first) {
     const GsCorners k = gs_corners(g.x, g.y, p);
     for (int c = c0; c < c1; ++c) {
-      const float go = gs_load(p.gout, (static_cast<int64_t>(n) * p.c + c) * p.points + pt, bf);
-      float* acc = gs_acc + (c - c0) * band_px - lo;
+      const float go = c == c0 ? go_first : gs_load(p.gout, go0 + static_cast<int64_t>(c - c0) * p.points + pt, bf);
+      double* acc = gs_acc + (c - c0) * band_px - lo;
       auto add = [&](int idx, float wt) {
-        if (wt != 0.0f && idx >= lo && idx < hi) atomicAdd(acc + idx, wt * go);
+        if (wt != 0.0f && idx >= lo && idx < hi) atomicAdd(acc + idx, static_cast<double>(wt * go));
       };
       add(k.c00, k.w00);
       if (!p.nearest) {
@@ -235,12 +276,29 @@ __global__ void __launch_bounds__(256) gs_bwd_input_kernel(const GridSampleParam
         add(k.c11, k.w11);
       }
     }
-  }
+  };
+#pragma unroll
+  for (int u = 0; u < kGsAhead; ++u)
+    if (u * step < left) scatter(first + u * step, ahead[u], go_ahead[u]);
+  for (uint32_t o = kGsAhead * step; o < left; o += step) scatter(first + o, grid[first + o], gs_load(p.gout, go0 + first + o, bf));
   __syncthreads();
-  const int64_t plane = static_cast<int64_t>(p.h) * w;
-  for (int i = threadIdx.x; i < cells; i += blockDim.x) {
-    const int cc = i / band_px, px = i - cc * band_px;
-    gs_store(p.ginput, (static_cast<int64_t>(n) * p.c + c0 + cc) * plane + lo + px, gs_acc[i], bf);
+  // the chunk's planes in one run of lanes (a band may be shorter than the workgroup)
+  const int64_t plane = static_cast<int64_t>(p.h) * w, out0 = (static_cast<int64_t>(n) * p.c + c0) * plane + lo;
+  const bool one = c1 - c0 == 1;
+  if (vec) {
+    const int quads = band_px / 4;
+    float* out = static_cast<float*>(p.ginput) + out0;
+    for (int i = threadIdx.x; i < cells / 4; i += blockDim.x) {
+      const int cc = one ? 0 : i / quads;
+      const double2 a = reinterpret_cast<const double2*>(gs_acc)[2 * i], b = reinterpret_cast<const double2*>(gs_acc)[2 * i + 1];
+      reinterpret_cast<float4*>(out + cc * plane)[i - cc * quads] =
+          make_float4(static_cast<float>(a.x), static_cast<float>(a.y), static_cast<float>(b.x), static_cast<float>(b.y));
+    }
+  } else {
+    for (int i = threadIdx.x; i < cells; i += blockDim.x) {
+      const int cc = one ? 0 : i / band_px;
+      gs_store(p.ginput, out0 + cc * plane + (i - cc * band_px), static_cast<float>(gs_acc[i]), bf);
+    }
   }
 }
 

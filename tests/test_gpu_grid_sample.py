@@ -173,3 +173,38 @@ def test_forward_paths_agree(tune, staged):
         out = hip.point_sample(_t(inputs), _t(pts), mode)
         want = GS.point_sample(inputs, pts, mode)
         assert_close(_np(out), want, 1e-5, f"{mode} staged={staged}")
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+@pytest.mark.parametrize("n,c,h,w,points", [
+    (1, 1, 3, 16384, 40),      # the widest accepted row: one row of the accumulator is 128 KB
+    (1, 2, 5, 8196, 33),       # one row just past 64 KB, bands of one row
+    (3, 5, 37, 53, 513),       # odd rows, several channels per chunk, one point past a workgroup
+    (2, 20, 24, 28, 64),       # rows of quads, a last chunk with fewer channels
+    (1, 1, 112, 112, 4100),    # points past the ones requested ahead, one workgroup's share past 2048
+    (300, 1, 20, 24, 1),       # more slices than compute units, one point each
+])
+def test_bands_chunks_and_many_points(n, c, h, w, points, bf16):
+    """Workgroup edges of the staged forward and of grad_input against the float64 oracle, with the
+    tolerances of this file; points lie on and past the border too."""
+    rng = np.random.default_rng(5)
+    _note(f"grid sample edges N={n} C={c} {h}x{w} P={points} bf16={bf16}")
+    inputs = rng.standard_normal((n, c, h, w)).astype(np.float32)
+    grid = rng.uniform(-1.1, 1.1, (n, 1, points, 2)).astype(np.float32)
+    grid[:, :, ::7, 0] = 1.0
+    grad = rng.standard_normal((n, c, 1, points)).astype(np.float32)
+    dt = torch.bfloat16 if bf16 else torch.float32
+    ti, tr = _t(inputs).to(dt).requires_grad_(), _t(grad).to(dt)
+    inputs, grad = _np(ti), _np(tr)
+    out = hip.bilinear_grid_sample(ti, _t(grid), "zeros")
+    out.backward(tr)
+    assert_close(_np(out), GS.bilinear_grid_sample(inputs, grid, "zeros"), 2e-2 if bf16 else 1e-5, "out")
+    gi, _ = GS.grid_sample_vjp(inputs, grid, grad, "zeros")
+    assert_close(_np(ti.grad), gi, 2e-2 if bf16 else 1e-4, "grad_inputs")
+
+
+def test_too_wide_for_the_accumulator_is_refused():
+    v = torch.zeros((1, 1, 1, 16385), device=_dev())
+    with pytest.raises(Exception, match="width 16385"):
+        hip.grid_sample_backward(v, torch.zeros((1, 1, 2), device=_dev()), torch.zeros((1, 1, 1), device=_dev()), 0, 0, 0,
+                                 needs=(True, False))
