@@ -22,7 +22,7 @@
 // Measured (graph replays, f32, before -> after; relative 2-norm against float64 of the output and
 // of grad_q, grad_k, grad_v):
 //   104 slices x 8 heads, 300 x 32: forward 129 -> 76 us, backward 319 -> 238; 3.1e-7 -> 2.1e-7,
-//     4.8, 5.5, 5.5e-7 -> 4.3, 4.1, 4.2e-7
+//     4.8, 5.5, 5.5e-7 -> 2.3, 2.0, 1.9e-7
 //   32 x 8, 300 x 32: 44.6 -> 25, 88 -> 69;  2 x 8: 17.1 -> 12, 78 -> 52;  52 x 8, 128 x 32: 15.0 -> 12, 41 -> 37
 //   4 x 8, 600 x 32: forward 32.3 -> 20;  8 x 8, 300 x 64: 30.5 -> 21
 #pragma once
@@ -354,8 +354,16 @@ __global__ void __launch_bounds__(64 * RB, D == 32 ? 3 : 2) attn_fwd_split_kerne
     for (int nd = 0; nd < ND; ++nd) at_store_block<float>(op + 32 * nd, p.st[kAtO][3], qb * 32, L, o[nd], 1.0f, at_lds + wave * (at_scratch_bytes<float>() / 4), lane);
     if (qv && grp == 0) {
       float* stats = p.stats + (static_cast<int64_t>(w.zh) * L + qi) * 4;
-      stats[0] = m;
-      stats[1] = log2f(l);
+      // The weights sum to l = 2^e f, f in [1, 2): m + e, and log2 f with what m + e rounds off. The
+      // backward's s - stats[0] - stats[1] is then rounded at the size of the weight's own log2; with m
+      // and log2 l (3 to 24) the rounding of these was most of the gradients' error against float64:
+      // 300 x 32 4.3, 4.1, 4.2e-7 (grad_q, grad_k, grad_v) -> 2.3, 2.0, 1.9e-7; 50 x 32 3.0 -> 1.7e-7;
+      // 300 x 64 (backward on f32 MFMAs) 5.7, 6.0, 5.8e-7 -> 4.4, 4.7, 4.5e-7.
+      const float e = static_cast<float>(static_cast<int>(__float_as_uint(l) >> 23) - 127);
+      const float f = __uint_as_float((__float_as_uint(l) & 0x007fffffu) | 0x3f800000u);
+      const float me = m + e, t = me - m;
+      stats[0] = me;
+      stats[1] = log2f(f) + ((m - (me - t)) + (e - t));
     }
   }
 }

@@ -670,3 +670,23 @@ def test_split_operands_nonfinite(tune, where, value):
         assert np.array_equal(fine, np.isfinite(a)), name
         assert np.array_equal(np.isnan(a), np.isnan(b)), name
         np.testing.assert_allclose(a[fine], b[fine], rtol=1e-4, atol=1e-5 * max(1.0, np.abs(b[fine]).max()))
+
+
+@pytest.mark.parametrize("shape", [(2, 2, 1, 32), (2, 2, 50, 32), (1, 2, 300, 32), (2, 1, 62, 64), (1, 1, 600, 64)], ids=str)
+def test_split_forward_statistics(shape):
+    """The f32 forward's statistics: entry 0 + entry 1 is log2 of the sum of 2^x, and entry 1 (log2 of a sum in
+    [1, 2) and what entry 0 rounds off, at most 2^-20 for entries below 16) is small, so that a backward's x -
+    entry 0 - entry 1 is rounded at its own size. Bound: 32 sums a row and chunk of 2^-24 of the sum each, in log2
+    units 2.8e-6, and as much for the scores (64 products of 2^-22 of a score of 8 at most, mostly far below)."""
+    b, h, length, d = shape
+    _note(f"split forward statistics {shape}")
+    rng = np.random.default_rng(91 + length)
+    q, k, v = (rng.standard_normal((b, h, length, d)).astype(np.float32) for _ in range(3))
+    lay = _Layout(b, 1, h, length, d)
+    _, stats = attention_forward(_t(q), _t(k), _t(v), lay, lay.strides_bhld)
+    torch.cuda.synchronize()
+    st = _np(stats).reshape(b, h, length, 4).astype(np.float64)
+    x = np.einsum("bhqd,bhkd->bhqk", q.astype(np.float64), k.astype(np.float64)) * (np.log2(np.e) / np.sqrt(d))
+    want = x.max(-1) + np.log2(np.exp2(x - x.max(-1, keepdims=True)).sum(-1))
+    assert np.abs(st[..., 0] + st[..., 1] - want).max() <= 5.6e-6
+    assert st[..., 1].min() >= -(2.0 ** -20) and st[..., 1].max() <= 1.0 + 2.0 ** -20
