@@ -679,6 +679,8 @@ def test_split_forward_statistics(shape):
     entry 0 - entry 1 is rounded at its own size. Bound: 32 sums a row and chunk of 2^-24 of the sum each, in log2
     units 2.8e-6, and as much for the scores (64 products of 2^-22 of a score of 8 at most, mostly far below)."""
     b, h, length, d = shape
+    from rfdetr_jax_amd.attention import _Layout, attention_forward
+
     _note(f"split forward statistics {shape}")
     rng = np.random.default_rng(91 + length)
     q, k, v = (rng.standard_normal((b, h, length, d)).astype(np.float32) for _ in range(3))
