@@ -21,7 +21,7 @@
 //
 // Measured (graph replays, f32, before -> after; relative 2-norm against float64 of the output and
 // of grad_q, grad_k, grad_v):
-//   104 slices x 8 heads, 300 x 32: forward 129 -> 76 us, backward 319 -> 238; 3.1e-7 -> 2.1e-7,
+//   104 slices x 8 heads, 300 x 32: forward 129 -> 76 us, backward 319 -> 222; 3.1e-7 -> 2.1e-7,
 //     4.8, 5.5, 5.5e-7 -> 2.3, 2.0, 1.9e-7
 //   32 x 8, 300 x 32: 44.6 -> 25, 88 -> 69;  2 x 8: 17.1 -> 12, 78 -> 52;  52 x 8, 128 x 32: 15.0 -> 12, 41 -> 37
 //   4 x 8, 600 x 32: forward 32.3 -> 20;  8 x 8, 300 x 64: 30.5 -> 21
@@ -472,6 +472,12 @@ __device__ __forceinline__ void at_operand_tr(at_bf8 (&a)[kAtTerms], const uint1
 // two barriers of a phase the key waves write their tiles, and dV, dK and the next block's scores
 // overlap the dQ waves' products. The query rows have three buffers: the dQ waves write one while
 // key waves may still read the two before it.
+// A key wave's vector work is asked between its MFMAs where it does not depend on them: the softmax
+// weights beside dP's products, the split of the weights beside dK's (left to the compiler each came
+// after its MFMAs, and the three waves of a SIMD are in the same stage; also 8 registers spilled instead
+// of 15): 104 slices x 8 heads of 300 rows 228 -> 222 us. dV's products moved before the barriers, beside
+// the split of dS, took 236 to 243 (24 registers spilled).
+constexpr int kAtSchedReads = 0x100;  // __builtin_amdgcn_sched_barrier: only LDS reads may cross
 constexpr int kAtSplitRow = 32 * 32;  // elements of one term of a 32-row tile
 constexpr int at_fused_split_lds_bytes(int nb) {
   return 3 * (2 * kAtTerms * kAtSplitRow * 2 + 3 * 32 * 4) + 16 + 2 * nb * kAtTerms * kAtSplitRow * 2;
@@ -521,23 +527,27 @@ __global__ void __launch_bounds__(64 * (kAtFusedBlocks + 2), 3) attn_bwd_fused_s
       const uint16_t* Gb = Gt + b * kAtTerms * TR;
       if (kb == 0 && lane < 32 && j * 32 + lane < L)  // rowsum(dO * O) into the statistics (their entry 2)
         p.stats[(static_cast<int64_t>(zh) * L + j * 32 + lane) * 4 + 2] = Ds[32 * b + lane];
-      at_f16 s = at_scores_split<D>(Qb, TR, 0, kt, col, grp);         // S = Q K^T
+      at_f16 s = at_scores_split<D>(Qb, TR, 0, kt, col, grp);  // S = Q K^T
+      __builtin_amdgcn_sched_barrier(kAtSchedReads);
       const at_f16 dp = at_scores_split<D>(Gb, TR, 0, vt, col, grp);  // dP = dO V^T
       at_f16 pw;
 #pragma unroll
       for (int c4 = 0; c4 < 4; ++c4) {
         const int ql = 8 * c4 + 4 * grp;
         const at_f4 ms0 = *reinterpret_cast<const at_f4*>(&Ms[64 * b + 2 * ql]), ms1 = *reinterpret_cast<const at_f4*>(&Ms[64 * b + 2 * ql + 4]);
-        const at_f4 dd = *reinterpret_cast<const at_f4*>(&Ds[32 * b + ql]);
         const float mq[4] = {ms0[0], ms0[2], ms1[0], ms1[2]}, lq[4] = {ms0[1], ms0[3], ms1[1], ms1[3]};
+        // a lane past L holds the clamped last key: finite weights, and its rows of the key copy
+        // are 0, so it adds nothing to dQ; rows past L have m = +inf: weight 0
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          const int i = 4 * c4 + jj;
-          // a lane past L holds the clamped last key: finite weights, and its rows of the key copy
-          // are 0, so it adds nothing to dQ; rows past L have m = +inf: weight 0
-          pw[i] = at_exp2(fmaf(s[i], p.scale2, -mq[jj]) - lq[jj]);
-          s[i] = pw[i] * (dp[i] - dd[jj]);  // dS
-        }
+        for (int jj = 0; jj < 4; ++jj) pw[4 * c4 + jj] = at_exp2(fmaf(s[4 * c4 + jj], p.scale2, -mq[jj]) - lq[jj]);
+      }
+      at_interleave<12, 5>();
+      __builtin_amdgcn_sched_barrier(kAtSchedReads);
+#pragma unroll
+      for (int c4 = 0; c4 < 4; ++c4) {
+        const at_f4 dd = *reinterpret_cast<const at_f4*>(&Ds[32 * b + 8 * c4 + 4 * grp]);
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) s[4 * c4 + jj] = pw[4 * c4 + jj] * (dp[4 * c4 + jj] - dd[jj]);  // dS
       }
       at_bf8 ds[2][kAtTerms];
       at_split_regs(s, 0, ds[0]);
@@ -554,6 +564,7 @@ __global__ void __launch_bounds__(64 * (kAtFusedBlocks + 2), 3) attn_bwd_fused_s
         }
       __syncthreads();  // the block's tiles are written
       // dK^T += Q^T dS and dV^T += dO^T P: the block's sums by themselves, then added
+      at_bf8 pt[2][kAtTerms];
       {
         at_f16 acc = at_zero16();
         at_bf8 a0[kAtTerms], a1[kAtTerms];
@@ -563,13 +574,15 @@ __global__ void __launch_bounds__(64 * (kAtFusedBlocks + 2), 3) attn_bwd_fused_s
         at_mfma_small(acc, a1, ds[1]);
         at_mfma(acc, a0[0], ds[0][0]);
         at_mfma(acc, a1[0], ds[1][0]);
-        dk += acc;
-      }
-      {
-        at_f16 acc = at_zero16();
-        at_bf8 pt[2][kAtTerms], a0[kAtTerms], a1[kAtTerms];
         at_split_regs(pw, 0, pt[0]);
         at_split_regs(pw, 8, pt[1]);
+        at_interleave<12, 8>();
+        dk += acc;
+      }
+      __builtin_amdgcn_sched_barrier(kAtSchedReads);
+      {
+        at_f16 acc = at_zero16();
+        at_bf8 a0[kAtTerms], a1[kAtTerms];
         at_operand_tr<D>(a0, Gb, TR, 0, 0, 0, lane);
         at_operand_tr<D>(a1, Gb, TR, 0, 0, 1, lane);
         at_mfma_small(acc, a0, pt[0]);
