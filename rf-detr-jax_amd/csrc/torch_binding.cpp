@@ -193,6 +193,16 @@ Tensor like_if(bool wanted, const Tensor& t) { return wanted ? at::empty_like(t,
 // the cotangent of an output, in the type and layout that the kernels read
 Tensor cotangent(const Tensor& g, at::ScalarType type) { return g.to(type).contiguous(); }
 
+// A saved tensor in the type and layout that the kernels read. Hooks on saved tensors (offloading,
+// compression) hand back tensors of their own making: the values may come in another layout or type,
+// and anything else that the kernels would read past is refused (saved_as).
+Tensor restored(const Tensor& t, at::ScalarType type) {
+  TORCH_CHECK(t.defined() && t.is_cuda(), "a saved tensor came back on another device than the GPU; the HIP kernels need GPU tensors");
+  return t.scalar_type() == type && t.is_contiguous() ? t : t.to(type).contiguous();
+}
+
+void saved_as(bool expected) { TORCH_CHECK_VALUE(expected, "saved tensors came back with other shapes, or on other devices, than they were saved"); }
+
 // ---- the deformable-attention core ------------------------------------------------------------
 
 struct Core : torch::autograd::Function<Core> {
@@ -206,18 +216,20 @@ struct Core : torch::autograd::Function<Core> {
                                             d.positions, st);
     });
     ctx->save_for_backward({value, loc, attn});
-    ctx->saved_data["shapes"] = std::vector<int64_t>(d.shapes.begin(), d.shapes.end());
+    ctx->saved_data["shapes"] = shapes_and_type(d, value);
     ctx->saved_data["sampler"] = sampler;
     return out;
   }
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor &value = saved[0], &loc = saved[1], &attn = saved[2];
     const int64_t sampler = ctx->saved_data["sampler"].toInt();
+    Levels lv;
     Dims d;
-    shapes_of(ctx, value, loc, d);
+    const Tensor value = restored(saved[0], shapes_of(ctx, lv)), loc = restored(saved[1], at::kFloat), attn = restored(saved[2], at::kFloat);
     const Tensor g = cotangent(grads[0], at::kFloat);
+    saved_as(dims_of(value, loc, attn, std::move(lv), d) && g.device() == value.device() &&
+             g.sizes().equals({d.batch, d.queries, int64_t{d.heads} * d.head_dim}));
     Tensor gv = like_if(ctx->needs_input_grad(0), value), gl = like_if(ctx->needs_input_grad(1), loc), ga = like_if(ctx->needs_input_grad(2), attn);
     Tensor ws;
     int64_t bytes = 0;
@@ -237,24 +249,22 @@ struct Core : torch::autograd::Function<Core> {
     return {gv, gl, ga, Tensor(), Tensor()};
   }
 
-  // the dims of a backward from its saved tensors
-  static void shapes_of(AutogradContext* ctx, const Tensor& value, const Tensor& samples, Dims& d) {
-    const auto s = samples.sizes();
-    d.batch = static_cast<int>(s[0]);
-    d.queries = static_cast<int>(s[1]);
-    d.heads = static_cast<int>(s[2]);
-    d.levels = static_cast<int>(s[3]);
-    d.points = static_cast<int>(s[4]);
-    d.head_dim = static_cast<int>(value.size(2));
-    d.positions = value.size(1);
-    int64_t at = 0;
-    const auto shapes = ctx->saved_data["shapes"].toIntVector();
-    for (size_t i = 0; i < shapes.size(); i += 2) {
-      d.shapes.push_back(static_cast<int32_t>(shapes[i]));
-      d.shapes.push_back(static_cast<int32_t>(shapes[i + 1]));
-      d.starts.push_back(static_cast<int32_t>(at));
-      at += shapes[i] * shapes[i + 1];
+  // the level shapes and the value type of a call, kept for its backward
+  static std::vector<int64_t> shapes_and_type(const Dims& d, const Tensor& value) {
+    std::vector<int64_t> kept(d.shapes.begin(), d.shapes.end());
+    kept.push_back(static_cast<int64_t>(value.scalar_type()));
+    return kept;
+  }
+
+  static at::ScalarType shapes_of(AutogradContext* ctx, Levels& lv) {
+    const auto kept = ctx->saved_data["shapes"].toIntVector();
+    for (size_t i = 0; i + 1 < kept.size(); i += 2) {
+      lv.shapes.push_back(static_cast<int32_t>(kept[i]));
+      lv.shapes.push_back(static_cast<int32_t>(kept[i + 1]));
+      lv.starts.push_back(static_cast<int32_t>(lv.positions));
+      lv.positions += kept[i] * kept[i + 1];
     }
+    return static_cast<at::ScalarType>(kept.back());
   }
 };
 
@@ -278,17 +288,20 @@ struct Fused : torch::autograd::Function<Fused> {
                            d.batch, d.heads, d.head_dim, d.queries, d.levels, d.points, d.shapes.data(), d.starts.data(), d.positions, st);
     });
     ctx->save_for_backward({value, ref, off, logits});
-    ctx->saved_data["shapes"] = std::vector<int64_t>(d.shapes.begin(), d.shapes.end());
+    ctx->saved_data["shapes"] = Core::shapes_and_type(d, value);
     return out;
   }
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor &value = saved[0], &ref = saved[1], &off = saved[2], &logits = saved[3];
+    Levels lv;
     Dims d;
-    Core::shapes_of(ctx, value, off, d);
-    const int ref_dim = static_cast<int>(ref.size(3));
+    const Tensor value = restored(saved[0], Core::shapes_of(ctx, lv)), ref = restored(saved[1], at::kFloat);
+    const Tensor off = restored(saved[2], at::kFloat), logits = restored(saved[3], at::kFloat);
     const Tensor g = cotangent(grads[0], at::kFloat);
+    saved_as(dims_of(value, off, logits, std::move(lv), d) && ref_matches(ref, value, d) && g.device() == value.device() &&
+             g.sizes().equals({d.batch, d.queries, int64_t{d.heads} * d.head_dim}));
+    const int ref_dim = static_cast<int>(ref.size(3));
     Tensor gv = like_if(ctx->needs_input_grad(0), value), gr = like_if(ctx->needs_input_grad(1), ref);
     Tensor go = like_if(ctx->needs_input_grad(2), off), gl = like_if(ctx->needs_input_grad(3), logits);
     const int64_t bytes = lib.fused_bwd_workspace_size(d.batch, d.heads, d.head_dim, d.queries, d.levels, d.points, ref_dim, d.shapes.data(),
@@ -302,6 +315,12 @@ struct Fused : torch::autograd::Function<Fused> {
     });
     return {gv, gr, go, gl, Tensor()};
   }
+
+  // reference points [B, Q, L, 2 | 4], contiguous
+  static bool ref_matches(const Tensor& ref, const Tensor& value, const Dims& d) {
+    return ref.dim() == 4 && f32(ref) && ref.is_contiguous() && ref.device() == value.device() && ref.size(0) == d.batch &&
+           ref.size(1) == d.queries && ref.size(2) == d.levels && (ref.size(3) == 2 || ref.size(3) == 4);
+  }
 };
 
 py::object fused(const py::handle& value, const py::handle& shapes, const py::handle& ref, const py::handle& off, const py::handle& logits) {
@@ -311,9 +330,7 @@ py::object fused(const py::handle& value, const py::handle& shapes, const py::ha
   if (!ordinary_state() || (v = plain(value)) == nullptr || (r = plain(ref)) == nullptr || (o = plain(off)) == nullptr ||
       (l = plain(logits)) == nullptr || !levels_of(shapes, lv) || !dims_of(*v, *o, *l, std::move(lv), d))
     return py::none();
-  if (r->dim() != 4 || !f32(*r) || !r->is_contiguous() || r->device() != v->device() || r->size(0) != d.batch || r->size(1) != d.queries ||
-      r->size(2) != d.levels || (r->size(3) != 2 && r->size(3) != 4))
-    return py::none();
+  if (!Fused::ref_matches(*r, *v, d)) return py::none();
   return py::cast(Fused::apply(*v, *r, *o, *l, d));
 }
 
@@ -337,8 +354,12 @@ struct ValueProj : torch::autograd::Function<ValueProj> {
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor &x = saved[0], &w = saved[1], &mask = saved[2];
+    const Tensor x = restored(saved[0], grads[0].scalar_type()), w = restored(saved[1], at::kFloat);
+    const Tensor mask = saved[2].defined() ? restored(saved[2], at::kBool) : Tensor();
     const int64_t heads = ctx->saved_data["heads"].toInt();
+    saved_as(x.dim() == 3 && w.dim() == 2 && w.size(1) == x.size(2) && w.size(0) % heads == 0 && w.device() == x.device() &&
+             grads[0].device() == x.device() && grads[0].sizes().equals({x.size(0) * heads, x.size(1), w.size(0) / heads}) &&
+             (!mask.defined() || (mask.device() == x.device() && mask.sizes().equals({x.size(0), x.size(1)}))));
     const int b = static_cast<int>(x.size(0)), s = static_cast<int>(x.size(1)), k = static_cast<int>(x.size(2)), h = static_cast<int>(heads);
     const int d = static_cast<int>(w.size(0) / heads);
     const Tensor g = cotangent(grads[0], x.scalar_type());
@@ -395,7 +416,9 @@ struct GridSample : torch::autograd::Function<GridSample> {
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor &in = saved[0], &grid = saved[1];
+    const Tensor in = restored(saved[0], grads[0].scalar_type()), grid = restored(saved[1], at::kFloat);
+    saved_as(in.dim() == 4 && grid.dim() == 3 && grid.size(0) == in.size(0) && grid.size(2) == 2 && grid.device() == in.device() &&
+             grads[0].device() == in.device() && grads[0].sizes().equals({in.size(0), in.size(1), grid.size(1)}));
     const auto modes = ctx->saved_data["modes"].toIntVector();
     const Tensor g = cotangent(grads[0], in.scalar_type());
     Tensor gi = like_if(ctx->needs_input_grad(0), in), gg = like_if(ctx->needs_input_grad(1), grid);
@@ -453,10 +476,19 @@ struct Attention : torch::autograd::Function<Attention> {
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &stats = saved[4];
+    const auto channels = [&](const Tensor& t) {  // any row strides
+      return t.defined() && t.is_cuda() && t.scalar_type() == grads[0].scalar_type() && t.dim() != 0 && t.stride(-1) == 1
+                 ? t
+                 : restored(t, grads[0].scalar_type());
+    };
+    const Tensor q = channels(saved[0]), k = channels(saved[1]), v = channels(saved[2]), out = channels(saved[3]);
+    const Tensor stats = restored(saved[4], at::kFloat);
     const auto n = ctx->saved_data["layout"].toIntVector();
     const Layout lay{static_cast<int>(n[0]), static_cast<int>(n[1]), static_cast<int>(n[2]), static_cast<int>(n[3]), static_cast<int>(n[4]), n[5] != 0};
-    Tensor g = grads[0].to(q.scalar_type());
+    for (const Tensor* t : {&q, &k, &v, &out}) saved_as(t->sizes() == grads[0].sizes() && t->device() == q.device());
+    saved_as(grads[0].device() == q.device() && stats.device() == q.device() &&
+             stats.numel() == int64_t{lay.batch} * lay.groups * lay.heads * lay.len * 4);
+    Tensor g = grads[0];
     if (g.stride(-1) != 1) g = g.contiguous();
     Tensor gq = like_if(ctx->needs_input_grad(0), q), gk = like_if(ctx->needs_input_grad(1), k), gv = like_if(ctx->needs_input_grad(2), v);
     int64_t st[32] = {};

@@ -195,6 +195,38 @@ def test_binding_saved_tensors(op):
         out.sum().backward()
 
 
+def _other_layout(t):
+    """The same values, channels first in memory."""
+    return t.movedim(-1, 0).contiguous().movedim(0, -1)
+
+
+@pytest.mark.parametrize("op", OPS)
+def test_binding_saved_tensor_hooks(op):
+    """What hooks make of the saved tensors reaches the kernels by its values: in another layout, or in
+    bfloat16 (as if rounded to it and brought back). Other shapes and CPU tensors are refused."""
+    fn, tensors = _call(op, torch.float32)
+
+    def grads(unpack):
+        ins = [t.detach().clone().requires_grad_() for t in tensors]
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            out = fn(*ins)
+        assert _is_binding(out, op)
+        torch.manual_seed(5)
+        return torch.autograd.grad(out, ins, _draw(*out.shape))
+
+    def floats(f):
+        return lambda t: f(t) if t.dtype == torch.float32 else t
+
+    want, rounded = grads(lambda t: t), grads(floats(lambda t: t.bfloat16().float()))
+    for got, expected in ((grads(_other_layout), want), (grads(floats(lambda t: t.bfloat16())), rounded)):
+        for a, b in zip(got, expected, strict=True):
+            assert a.dtype == b.dtype
+            torch.testing.assert_close(a, b, rtol=1e-6, atol=1e-6)
+    for wrong in (lambda t: t[..., :-1], lambda t: t[None], lambda t: t.cpu()):
+        with pytest.raises((ValueError, RuntimeError), match="saved tensor|invalid gradient"):
+            grads(wrong)
+
+
 def test_binding_errors_keep_their_type():
     """A shape that only the library refuses raises MsdaError from the forward and from the backward."""
     q = _draw(1, 1, 8, 48)  # head_dim 48
