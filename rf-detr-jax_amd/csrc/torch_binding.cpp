@@ -182,8 +182,9 @@ bool dims_of(const Tensor& value, const Tensor& samples, const Tensor& weights, 
   return true;
 }
 
+// at least `bytes`, in whole 16-byte rows
 Tensor workspace(int64_t bytes, const Tensor& like) {
-  return at::empty({std::max<int64_t>(1, bytes / 16), 4}, like.options().dtype(at::kInt));
+  return at::empty({std::max<int64_t>(1, (bytes + 15) / 16), 4}, like.options().dtype(at::kInt));
 }
 
 void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
@@ -532,6 +533,7 @@ PYBIND11_MODULE(_torch_binding, m) {
     }
   });
   m.def("bind", &bind);
+  m.def("workspace", &workspace);
   m.def("core", &core);
   m.def("fused", &fused);
   m.def("value_proj", &value_proj);

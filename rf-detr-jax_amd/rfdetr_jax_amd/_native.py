@@ -133,6 +133,12 @@ def check(rc: int) -> None:
         raise MsdaError(rc, msg)
 
 
+def workspace(nbytes: int, device) -> torch.Tensor:
+    """Scratch memory of at least ``nbytes`` (16-byte aligned, in whole 16-byte rows); torch's caching
+    allocator serves it."""
+    return torch.empty((max(1, (nbytes + 15) // 16), 4), dtype=torch.int32, device=device)
+
+
 @contextlib.contextmanager
 def tuning(knobs: dict):
     """Override launch-tuning knobs (``{"MSDA_BWD_BANDS": 7, ...}``) for the duration of a block;

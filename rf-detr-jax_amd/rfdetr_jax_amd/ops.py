@@ -192,8 +192,7 @@ def ms_deform_attn_backward(value, spatial_shapes, sampling_locations, attention
         ws_bytes = lib.msda_bwd_workspace_size(*dims)
         if ws_bytes < 0:
             _native.check(int(ws_bytes))
-        # the query blocks' partial grad_value sums (f32); torch's caching allocator serves it
-        workspace = torch.empty((max(1, ws_bytes // 16), 4), dtype=torch.int32, device=dev)
+        workspace = _native.workspace(ws_bytes, dev)  # the query blocks' partial grad_value sums (f32)
     with torch.cuda.device(dev):
         head = (_ptr(value), _VALUE_DTYPES[value.dtype], _ptr(loc), _ptr(attn), _ptr(grad_output),
                 _VALUE_DTYPES[grad_output.dtype], _ptr(grad_value), _ptr(grad_loc), _ptr(grad_attn))
@@ -362,7 +361,7 @@ def ms_deform_attn_fused_backward(value, spatial_shapes, reference_points, sampl
                                                  starts, value.shape[1])
     if ws_bytes < 0:
         _native.check(int(ws_bytes))
-    workspace = torch.empty((max(1, ws_bytes // 16), 4), dtype=torch.int32, device=dev)
+    workspace = _native.workspace(ws_bytes, dev)
     with torch.cuda.device(dev):
         rc = lib.msda_fused_bwd(
             _ptr(value), _VALUE_DTYPES[value.dtype], _ptr(ref), ref_dim, _ptr(off), _ptr(logits), _ptr(grad_output),

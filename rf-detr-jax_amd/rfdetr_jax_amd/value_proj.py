@@ -87,7 +87,7 @@ def value_proj_backward(x, weight, n_heads, grad_value, padding_mask=None, needs
         ws = lib.msda_value_proj_bwd_workspace_size(b, s, k, n_heads, d)
         if ws < 0:
             _native.check(int(ws))
-        workspace = torch.empty((max(1, ws // 16), 4), dtype=torch.int32, device=x.device)
+        workspace = _native.workspace(ws, x.device)
     with torch.cuda.device(x.device):
         rc = lib.msda_value_proj_bwd(_ptr(x), _DTYPES[x.dtype], _ptr(w), _ptr(mask), _ptr(gv), _ptr(gx), _ptr(gw), _ptr(gb), b, s, k,
                                      n_heads, d, _ptr(workspace), ws, _stream(x.device))

@@ -454,6 +454,15 @@ def test_value_proj_workspace():
     assert _vp_fwd(batch=0)[0] == _native.OK
 
 
+@pytest.mark.parametrize("heads, dim, features", [(1, 1, 64), (1, 2, 64), (1, 3, 64), (3, 1, 5), (2, 16, 32)])
+def test_front_ends_allocate_the_whole_workspace(heads, dim, features):
+    """Both front-ends' buffers hold every byte of a size that is not a multiple of their 16-byte rows."""
+    size = _native.lib().msda_value_proj_bwd_workspace_size(1, 40, features, heads, dim)
+    assert size == heads * dim * (features + 1) * 4
+    for ws in (_native.workspace(size, "cpu"), _native.binding().workspace(size, torch.empty(1))):
+        assert ws.numel() * ws.element_size() >= size
+
+
 def test_ms_deform_attn_module_mirror_errors():
     from rfdetr_jax_amd import MSDeformAttn
     from rfdetr_jax_amd.value_proj import value_proj_rows
