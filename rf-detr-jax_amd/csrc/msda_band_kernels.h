@@ -93,8 +93,11 @@ struct BandItem {
 };
 
 __device__ __forceinline__ BandItem band_item(const BandParams& p, int k) {
+  // 64-bit: another level may have more items (1e5 of a row each) than this one's band has rows to spare
+  // below 2^31
+  auto past = [&](const LevelDesc& v) { return static_cast<int64_t>(k - v.band_first) * v.band_rows >= v.h; };
   int l = 0;
-  while (l + 1 < p.levels && (k < p.lv[l].band_first || (k - p.lv[l].band_first) * p.lv[l].band_rows >= p.lv[l].h)) ++l;
+  while (l + 1 < p.levels && (k < p.lv[l].band_first || past(p.lv[l]))) ++l;
   BandItem it;
   it.l = l;
   it.r0 = (k - p.lv[l].band_first) * p.lv[l].band_rows;

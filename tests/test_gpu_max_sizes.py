@@ -14,6 +14,7 @@ the size:
   and in the weights, so <G, out> = <dV, V> = <dA, A> (sums in float64 on the GPU);
 * a level too wide for one image row of the backward's f64 accumulator to fit in LDS is refused
   with MSDA_ERR_UNSUPPORTED, its forward still runs;
+* the backward with 160000 one-row bands beside one band of 13600 rows (item number x rows passes 2^31);
 * a level whose image row fits only beside a shorter point list (more scan passes per band)
   against the float64 oracle;
 * the self-attention at 2048 and 4096 rows against the float64 oracle.
@@ -114,6 +115,39 @@ def test_level_too_wide_for_the_backward_is_refused():
         hip.ms_deform_attn_backward(value, shapes, loc, attn, grad)
     assert err.value.code == _native.ERR_UNSUPPORTED
     _note(f"refused: {err.value}")
+
+
+def test_many_bands_beside_a_tall_one():
+    """Five levels of 32000 one-row bands after a one-column level that is one band of 13600 rows: the last
+    bands' item numbers times its rows pass 2^31. On a constant value map, grad_value sums to the weighted
+    cotangents, within the rows that the samples touch, and grad_attn is the constant times the cotangent."""
+    h, w, q = 32000, 5840, 64
+    shapes = ((13600, 1),) + ((h, w),) * 5
+    assert 32000 * 5 * 13600 >= 1 << 31
+    _note(f"max size band items {shapes}")
+    dev = torch.device("cuda:0")
+    gen = _gen(13)
+    value = torch.full((1, sum(a * b for a, b in shapes), 1), 2.0, device=dev)
+    loc = 0.1 + 0.8 * torch.rand(1, q, 1, len(shapes), 1, 2, device=dev, generator=gen)
+    loc[:, :, :, 0, :, 0] = 0.5  # on the one column: beside it the zero padding takes a share of the weight
+    loc[:, :, :, 1:, :, 1] = 0.99 + 0.009 * torch.rand(1, q, 1, 5, 1, device=dev, generator=gen)  # the last bands
+    attn = torch.softmax(torch.randn(1, q, 1, len(shapes), device=dev, generator=gen), -1)
+    grad = torch.randn(1, q, 1, device=dev, generator=gen)
+    gv, _, ga = hip.ms_deform_attn_backward(value, shapes, loc, attn, grad)
+    torch.cuda.synchronize()
+    torch.testing.assert_close(ga, 2.0 * grad[..., None].expand_as(ga), rtol=0.0, atol=3e-4)  # weights of 2^-9 pixels
+    at = 0
+    for l, (lh, lw) in enumerate(shapes):
+        level = gv[0, at:at + lh * lw, 0].view(lh, lw)
+        at += lh * lw
+        want = float((attn[0, :, 0, l].double() * grad[0, :, 0].double()).sum())
+        assert abs(float(level.double().sum()) - want) <= 1e-4, l
+        rows = level.abs().sum(1).nonzero()[:, 0]
+        y = loc[0, :, 0, l, 0, 1].double() * lh - 0.5
+        near = (rows[:, None].double() - y[None]).abs().amin(1)
+        assert len(rows) > 0 and float(near.max()) <= 1.01, l
+        assert float((y[None] - rows[:, None].double()).abs().amin(0).max()) <= 1.01, l
+    del value, gv
 
 
 def test_wide_level_with_a_shorter_point_list_against_oracle():
