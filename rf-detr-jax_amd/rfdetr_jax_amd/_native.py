@@ -11,6 +11,7 @@ import ctypes
 import importlib.util
 import os
 import threading
+import warnings
 
 import torch
 
@@ -82,6 +83,10 @@ class MsdaError(RuntimeError):
         self.code = code
 
 
+def _library_path() -> str:
+    return os.environ.get("MSDA_LIBRARY", LIB_PATH)
+
+
 def lib(path: str | None = None) -> ctypes.CDLL:
     """Load (once) and return the HIP library."""
     global _lib
@@ -90,7 +95,7 @@ def lib(path: str | None = None) -> ctypes.CDLL:
     with _lock:
         if _lib is not None and path is None:
             return _lib
-        target = path or os.environ.get("MSDA_LIBRARY", LIB_PATH)
+        target = path or _library_path()
         if not os.path.exists(target):
             raise RuntimeError(
                 f"HIP library not found at {target}; build it with __graft_entry__.build() "
@@ -106,21 +111,35 @@ def lib(path: str | None = None) -> ctypes.CDLL:
         return handle
 
 
+class _NoBinding:
+    """Leaves every call to the Python autograd functions."""
+
+    core = fused = value_proj = grid_sample = attention = staticmethod(lambda *args: None)
+
+
 def binding():
     """Load (once) and return the torch binding: the differentiable ops as C++ autograd functions over
-    the library's C ABI, each returning None for a call that the Python path has to take."""
+    the library's C ABI, each returning None for a call that the Python path has to take. Without the
+    library the Python path reports what is missing; without the binding, which only saves host time,
+    it takes every call."""
     global _binding
     if _binding is not None:
         return _binding
+    if _lib is None and not os.path.exists(_library_path()):
+        return _NoBinding
     handle = lib()
     with _lock:
         if _binding is not None:
             return _binding
-        if not os.path.exists(BINDING_PATH):
-            raise RuntimeError(f"torch binding not found at {BINDING_PATH}; build it with __graft_entry__.build()")
-        spec = importlib.util.spec_from_file_location("rfdetr_jax_amd._torch_binding", BINDING_PATH)
-        module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(module)
+        try:
+            spec = importlib.util.spec_from_file_location("rfdetr_jax_amd._torch_binding", BINDING_PATH)
+            module = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(module)
+        except ImportError as e:  # not built, or built against another torch
+            warnings.warn(f"the torch binding at {BINDING_PATH} does not load ({e}); every call takes the slower Python path. "
+                          "Build it with __graft_entry__.build().", RuntimeWarning, stacklevel=3)
+            _binding = _NoBinding
+            return _binding
         address = {name: ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in SIGNATURES}
         module.bind(address, check, torch.nn.Parameter)
         _binding = module

@@ -13,6 +13,7 @@ import ctypes
 import glob
 import os
 import re
+import warnings
 
 import pytest
 import torch
@@ -603,3 +604,31 @@ def test_attention_dropout_keep_validation():
     assert lib.msda_attention_dropout_keep(2, 1, 2, -1, 0.1, 1, None, None) == _native.ERR_INVALID_ARGUMENT
     assert lib.msda_attention_dropout_keep(2, 1, 2, 9, 0.1, 1, None, None) == _native.ERR_INVALID_ARGUMENT  # NULL keep
     assert lib.msda_attention_dropout_keep(2, 1, 2, 0, 0.1, 1, None, None) == _native.OK
+
+
+def _rows(*shape):
+    return torch.zeros(shape), ((2, 2),), torch.zeros(1, 3, 2, 1, 1, 2), torch.zeros(1, 3, 2, 1)
+
+
+def test_front_end_without_the_binding(monkeypatch, tmp_path):
+    """A tree with the library alone still runs: the Python functions take every call (here up to their
+    checks), after one warning."""
+    monkeypatch.setattr(_native, "_binding", None)
+    monkeypatch.setattr(_native, "BINDING_PATH", str(tmp_path / "_torch_binding.so"))
+    with pytest.warns(RuntimeWarning, match="Python path"), pytest.raises(RuntimeError, match="GPU tensors"):
+        hip_ops.ms_deform_attn_core_rows(*_rows(2, 4, 8))
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        with pytest.raises(ValueError, match="value length 5"):
+            hip_ops.ms_deform_attn_core_rows(*_rows(2, 5, 8))
+
+
+def test_front_end_checks_without_the_library(monkeypatch, tmp_path):
+    """Inconsistent shapes are reported as such, library or not; a call that needs it names it."""
+    monkeypatch.setattr(_native, "_binding", None)
+    monkeypatch.setattr(_native, "_lib", None)
+    monkeypatch.setenv("MSDA_LIBRARY", str(tmp_path / "libmsda.so"))
+    with pytest.raises(ValueError, match="value length 5"):
+        hip_ops.ms_deform_attn_core_rows(*_rows(2, 5, 8))
+    with pytest.raises(RuntimeError, match="HIP library not found"):
+        _native.lib()
