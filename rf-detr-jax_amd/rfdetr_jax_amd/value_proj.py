@@ -123,7 +123,7 @@ def value_proj_rows(x, weight, bias, n_heads, padding_mask=None):
         n_heads: number of heads.
         padding_mask: ``[B, S]`` bool, ``True`` on padded positions, or ``None``.
     """
-    if type(n_heads) is int:
+    if type(n_heads) is int and 0 < n_heads < 2 ** 31:  # others: the Python path's errors
         out = _native.binding().value_proj(x, weight, bias, n_heads, padding_mask)
         if out is not None:
             return out

@@ -21,6 +21,7 @@ import torch
 from rfdetr_jax_amd import _native
 from rfdetr_jax_amd import ops as hip_ops
 from rfdetr_jax_amd.build import LIB_PATH
+from rfdetr_jax_amd.value_proj import value_proj_rows
 
 INCLUDE = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "include")
 
@@ -632,3 +633,9 @@ def test_front_end_checks_without_the_library(monkeypatch, tmp_path):
         hip_ops.ms_deform_attn_core_rows(*_rows(2, 5, 8))
     with pytest.raises(RuntimeError, match="HIP library not found"):
         _native.lib()
+
+
+@pytest.mark.parametrize("n_heads", [3, 2 ** 31, 2 ** 70, -(2 ** 70)])
+def test_value_proj_refuses_head_counts_by_the_shape_check(n_heads):
+    with pytest.raises(ValueError, match="weight must be"):
+        value_proj_rows(torch.zeros(1, 2, 4), torch.zeros(8, 4), None, n_heads)
