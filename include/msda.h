@@ -364,11 +364,13 @@ int msda_value_proj_bwd(const void* input, int dtype, const float* weight, const
  *
  * mask: [len, len] bytes (non-zero blocks a key for a query: torch's boolean convention,
  * layers.py:69, :93-94) or NULL. dtype: MSDA_DTYPE_F32 or MSDA_DTYPE_BF16 for every tensor;
- * arithmetic is f32 (v_mfma_f32_32x32x2_f32), softmax in f32.
+ * sums and softmax are f32. f32 products run on f32 matrix instructions (v_mfma_f32_32x32x2_f32) with
+ * a mask or dropout, and otherwise on operands of three bf16 terms, which hold f32's 24 significand
+ * bits (attention_split_kernels.h); bf16 products run on bf16 matrix instructions.
  * stats: [batch * groups * heads * len][4] f32, 16-byte aligned, z-major (z = g * batch + b), then
- * head, then query: the forward writes entries 0 and 1 (a reference score m, between 8 below and
- * 64 above the row maximum, and log2 of the softmax denominator taken relative to m (at most a
- * rounding of m below 0), in units of log2(e) q.k / sqrt(D)); the backward reads them and uses entry 2 for rowsum(grad_out * out).
+ * head, then query: the forward writes entries 0 and 1, whose sum is log2 of the row's sum of 2^x over
+ * the keys, x = log2(e) q.k / sqrt(D) (entry 0 alone is within 64 of that sum); the backward reads them
+ * and uses entry 2 for rowsum(grad_out * out).
  * Dropout on the attention weights (layers.py:537-544, active only with dropout > 0 in training)
  * is msda_attention_fwd_dropout's. len is at most 65536, each row stride s_row below 2^24 elements
  * and len * s_row below 2^31 (row offsets within a (slice, head) are formed in 32 bits).

@@ -94,8 +94,9 @@ int fwd_rb(const msda::AttnParams& p, hipStream_t st) {
   return at_launch(msda::attn_fwd_kernel<VT, D, MASK, RB, DROP>, granted, p, lds_bytes(D), RB, st, "attention forward");
 }
 
-// f32 with a mask or dropout runs on the f32 MFMAs, without on split f16 operands (300 x 32 rows, 104
-// slices x 8 heads: 129 -> 76 us; shorter and fewer rows gain too, 13 x 8 of 77 rows 9.0 -> 7.8).
+// f32 with a mask or dropout runs on the f32 MFMAs, without on operands of three bf16 terms (300 x 32
+// rows, 104 slices x 8 heads: 119 -> 84 us; no size is slower: 2 x 8 of 50 rows 5.8 both ways, 1 x 4 of
+// 2048 x 64 161 -> 105).
 template <int D>
 int fwd_f32(const msda::AttnParams& p, hipStream_t st) {
   static std::atomic<int> granted[msda_host::kMaxDevices];

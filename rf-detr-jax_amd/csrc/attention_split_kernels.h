@@ -2,29 +2,26 @@
 // a mask or dropout: the forward, and the fused backward (head_dim 32, up to 32 kAtFusedBlocks rows).
 //
 // v_mfma_f32_32x32x2_f32 takes 64 cycles for 4096 flops and bounded the f32 kernels
-// (attention_kernels.h). Here every operand, the softmax weights and dS included, is split into
-// 16-bit terms whose products run at 16 times that rate (10 times measured: dense 16-bit MFMAs reach
-// 1.6 PFLOP/s here); sums stay f32.
-//   * Backward: three bf16 terms, each the rounding of what the ones before left, hold all 24
-//     significand bits at any size a bf16 has, so gradients of any range split as well as any other;
-//     six products of terms t and u, t + u <= 2, the five small ones summed before the main one.
-//   * Forward: two f16 terms, h = f16(x) and l = f16(x - h), of values scaled into f16's range; h h +
-//     h l + l h. A scaled value is held to one unit of its 24th bit (exactly in three of four cases).
-//     Half the MFMAs and 2 vector operations per split value instead of 5.5: 76 us where three bf16
-//     terms took 100. Queries are scaled row by row; keys and values by the power of two that puts
-//     the largest element of the first 64 rows at 2^10. What could fall outside f16 then is checked,
-//     not assumed: a key or value beyond 65504, a channel of V whose largest element stays below
-//     2^-1 (its results would lose bits that the f32 kernel keeps), or a query and keys so large that
-//     what their small channels lose could show in the scores (kAtMaxProduct).
-// A workgroup that fails a check, or whose results are not all finite (an infinity leaves the split
-// as NaN), runs the f32 kernel's body instead.
+// (attention_kernels.h). Here every operand, the softmax weights and dS included, is split into three
+// bf16 terms, each the rounding of what the ones before left, which together hold the 24 significand
+// bits of a value of any size from 2^-109 up (below, to a unit of 2^-133). Of the products of terms t
+// and u the six with t + u <= 2 are summed, the five small ones before or beside the main one; what is
+// left out is below 2^-25 of a product, under the rounding of an f32 product. bf16 products run at 16
+// times the rate of f32 ones (10 times measured: dense bf16 MFMAs reach 1.6 PFLOP/s here); sums are f32.
+// A workgroup whose results are not all finite (an infinity, or a value that rounds to one in bf16,
+// leaves the split as NaN), and in the forward one that meets a non-zero element below 2^-100, does its
+// work again in the f32 kernel's body. Such a workgroup takes the time of both.
+// (Two f16 terms, scaled into f16's range, took 62 us where three bf16 terms take 84, and lost bits: the
+// low ones of a quarter of all values, and of rows far below the size that the scale was taken from,
+// with relative errors of 1e-2 at a spread of 1e8.)
 //
-// Measured (graph replays, f32, before -> after; relative 2-norm against float64 of the output and
-// of grad_q, grad_k, grad_v):
-//   104 slices x 8 heads, 300 x 32: forward 129 -> 76 us, backward 319 -> 222; 3.1e-7 -> 2.1e-7,
+// Measured (20 calls a graph, f32, f32 kernel -> these; relative 2-norm against float64 of the output
+// and of grad_q, grad_k, grad_v):
+//   104 slices x 8 heads, 300 x 32: forward 119 -> 84 us, backward 317 -> 228; 3.1e-7 -> 1.7e-7,
 //     4.8, 5.5, 5.5e-7 -> 2.3, 2.0, 1.9e-7
-//   32 x 8, 300 x 32: 44.6 -> 25, 88 -> 69;  2 x 8: 17.1 -> 12, 78 -> 52;  52 x 8, 128 x 32: 15.0 -> 12, 41 -> 37
-//   4 x 8, 600 x 32: forward 32.3 -> 20;  8 x 8, 300 x 64: 30.5 -> 21
+//   forward 32 x 8, 300 x 32: 40 -> 29;  2 x 8: 16.9 -> 13.6;  52 x 8, 128 x 32: 14.2 -> 12.6;  2 x 8, 50 x 32: 5.8, 5.8
+//   forward 4 x 8, 600 x 32: 30 -> 23;  104 x 4, 300 x 64: 119 -> 75;  8 x 8, 300 x 64: 29 -> 21.6
+//   backward 32 x 8, 300 x 32: 83 -> 63;  2 x 8: 78 -> 53;  52 x 8, 128 x 32: 39 -> 35
 #pragma once
 
 #include <type_traits>
@@ -33,342 +30,7 @@
 
 namespace msda {
 
-typedef _Float16 at_h8 __attribute__((ext_vector_type(8)));
-
-// a and b as packed f16 terms: w = f16(a) | f16(b) << 16 and its remainder r
-__device__ __forceinline__ void at_split2(float a, float b, uint32_t& w, uint32_t& r) {
-  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-  typedef float f2 __attribute__((ext_vector_type(2)));
-  w = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, h2));
-  float ra, rb;  // a - f16(a), exact
-  asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(ra) : "v"(w), "v"(a));
-  asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(rb) : "v"(w), "v"(b));
-  r = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{ra, rb}, h2));
-}
-
-struct AtH8 {  // an operand of eight values: terms h, l
-  at_h8 h, l;
-};
-
-__device__ __forceinline__ AtH8 at_split8(const at_f8& f) {
-  uint32_t w[4], r[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) at_split2(f[2 * i], f[2 * i + 1], w[i], r[i]);
-  return AtH8{__builtin_bit_cast(at_h8, uint4{w[0], w[1], w[2], w[3]}), __builtin_bit_cast(at_h8, uint4{r[0], r[1], r[2], r[3]})};
-}
-
-// result registers i0 .. i0 + 7
-__device__ __forceinline__ AtH8 at_split_regs(const at_f16& v, int i0) {
-  return at_split8(at_f8{v[i0], v[i0 + 1], v[i0 + 2], v[i0 + 3], v[i0 + 4], v[i0 + 5], v[i0 + 6], v[i0 + 7]});
-}
-
-__device__ __forceinline__ void at_mfma(at_f16& c, const at_h8& a, const at_h8& b) {
-  c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-
-// 2^k with k = 10 - floor(log2 max) (1 for 0; k at most 120), and its inverse
-__device__ __forceinline__ float at_pow2_scale(float max, float& inv) {
-  const int e = static_cast<int>((__float_as_uint(max) >> 23) & 255u);  // biased exponent
-  const int k = max == 0.0f ? 0 : min(137 - e, 120);
-  inv = __uint_as_float(static_cast<uint32_t>(127 - k) << 23);
-  return __uint_as_float(static_cast<uint32_t>(127 + k) << 23);
-}
-
-__device__ __forceinline__ float at_absmax4(const at_f4& v, float m) {
-  return fmaxf(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), m), fmaxf(fabsf(v[2]), fabsf(v[3])));
-}
-
-// Asks the scheduler to follow each of the block's N MFMAs by up to V vector operations: it would
-// issue the dependent MFMAs back to back and the vector work after them.
-template <int N, int V>
-__device__ __forceinline__ void at_interleave() {
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(0x2, V, 0);
-  }
-}
-
-// Term tiles: the rows of a chunk as swizzled f16 tiles [64][D] (at_swo), h then l.
-template <int D>
-__device__ __forceinline__ AtH8 at_tile_row(const uint16_t* X, int stride, int row, int ch) {  // channels ch .. ch + 7
-  const uint16_t* e = X + at_swo<D>(row, ch);
-  return AtH8{__builtin_bit_cast(at_h8, *reinterpret_cast<const uint4*>(e)), __builtin_bit_cast(at_h8, *reinterpret_cast<const uint4*>(e + stride))};
-}
-
-// Operand of X^T for MFMA (nd, s) of at_accum_tr: channel 32 nd + l % 32 at the rows of result
-// registers 8 s .. 8 s + 7, by transposing reads of the term tiles at row x.
-template <int D>
-__device__ __forceinline__ AtH8 at_tile_tr(const uint16_t* X, int stride, int x, int nd, int s, int lane) {
-  const int g = lane >> 4, r = lane & 15, grp = lane >> 5;
-  const int c = 32 * nd + 16 * (g & 1) + 4 * (r & 3), ro = x + 16 * s + 4 * grp + (r >> 2);
-  const int i0 = at_swo<D>(ro, c), i1 = at_swo<D>(ro + 8, c);
-  return AtH8{__builtin_bit_cast(at_h8, at_bf8_of(at_read_tr(X + i0), at_read_tr(X + i1))),
-              __builtin_bit_cast(at_h8, at_bf8_of(at_read_tr(X + stride + i0), at_read_tr(X + stride + i1)))};
-}
-
-// An AtChunk (64 f32 rows in registers) times `scale` as term tiles; rows past L are 0.
-template <int D, int NT>
-__device__ __forceinline__ void at_store_split(const AtChunk<float, D, NT>& ch, float scale, uint16_t* dst, int r0, int L) {
-#pragma unroll
-  for (int u = 0; u < AtChunk<float, D, NT>::NV; ++u) {
-    const int idx = threadIdx.x + NT * u, row = idx / (D / 4), c4 = idx - row * (D / 4);
-    const at_f4 v = ch.v[u] * (r0 + row < L ? scale : 0.0f);
-    uint2 h, l;
-    at_split2(v[0], v[1], h.x, l.x);
-    at_split2(v[2], v[3], h.y, l.y);
-    *reinterpret_cast<uint2*>(&dst[at_swo<D>(row, 4 * c4)]) = h;
-    *reinterpret_cast<uint2*>(&dst[kAtChunk * D + at_swo<D>(row, 4 * c4)]) = l;
-  }
-}
-
-constexpr float kAtF16Max = 65504.0f;
-// What scaling takes from a row's small channels moves a score by at most 2^-30 of max |q| max |k|:
-// f32's own rounding of a score while that product is within this bound (log2 units).
-constexpr float kAtMaxProduct = 256.0f;
-
-template <int D>
-constexpr int at_split_lds_bytes() { return 2 * 2 * 2 * kAtChunk * D * 2 + (4 * D + 4) * 4; }  // key and value term tiles, two buffers; reductions
-static_assert(at_split_lds_bytes<32>() >= at_lds_floats<32>() * 4 && at_split_lds_bytes<64>() >= at_lds_floats<64>() * 4, "the f32 body fits");
-
-// Forward (attn_fwd_kernel's work split and streaming). A workgroup splits each chunk once, into one
-// of two buffers in the shadow of the chunk before's MFMAs. The softmax reference m is moved when a
-// chunk's largest weight would leave [2^3, 2^15] (the first chunk) or exceed 2^15: the weights fit
-// f16, and what they lose below 2^-14 is 2^-28 of the row's largest.
-// Two workgroup-wide MFMA chains per key block pair; vector operations asked between the MFMAs of the
-// scores (10 each: 72 us; left to the compiler 81; 256 registers and two waves per SIMD instead of 168
-// and three: 77).
-template <int D, int RB>
-__global__ void __launch_bounds__(64 * RB, D == 32 ? 3 : 2) attn_fwd_split_kernel(const AttnParams p) {
-  constexpr int NT = 64 * RB, ND = D / 32, TS = kAtChunk * D;  // TS: elements of a term tile
-  extern __shared__ __align__(16) float at_lds[];
-  float* red = at_lds;  // [4][D], [4]
-  uint16_t* Kt = reinterpret_cast<uint16_t*>(at_lds + 4 * D + 4);
-  const int L = p.len, nb = (L + 31) / 32, nchunks = (L + kAtChunk - 1) / kAtChunk;
-  const AttnWork w(p, (nb + RB - 1) / RB);
-  const float* kp = static_cast<const float*>(p.k) + w.sl.base(p, kAtK);
-  const float* vp = static_cast<const float*>(p.v) + w.sl.base(p, kAtV);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, grp = lane >> 5, col = lane & 31;
-  const int qb = w.rc * RB + wave, qi = qb * 32 + col;
-  const bool qv = qi < L;
-  using Chunk = AtChunk<float, D, NT>;
-  Chunk kc, vc;
-  kc.load(kp, p.st[kAtK][3], 0, L);
-  vc.load(vp, p.st[kAtV][3], 0, L);
-  AtH8 qt[D / 16];
-  float iq, qm = 0.0f;  // what the query row was scaled by, inverse; its largest element
-  {
-    const float* qp = static_cast<const float*>(p.q) + w.sl.base(p, kAtQ) + at_row_off(min(qi, L - 1), p.st[kAtQ][3]);
-    at_f4 f[D / 16][2];
-#pragma unroll
-    for (int s = 0; s < D / 16; ++s)
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        f[s][u] = *reinterpret_cast<const at_f4*>(qp + 16 * s + 8 * grp + 4 * u);
-        qm = at_absmax4(f[s][u], qm);
-      }
-    qm = at_max_halves(qm);
-    const float sq = at_pow2_scale(qm, iq);
-#pragma unroll
-    for (int s = 0; s < D / 16; ++s) {
-      const at_f4 a = f[s][0] * sq, b = f[s][1] * sq;
-      qt[s] = at_split8(at_f8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]});
-    }
-  }
-  // largest |K| and |V| of the rows a thread stages (V: of its four channels), over the first chunk
-  // for the scales and over all chunks for the checks
-  float kmax = 0.0f;
-  at_f4 vmax = {0.0f, 0.0f, 0.0f, 0.0f};
-  auto track = [&] {
-#pragma unroll
-    for (int u = 0; u < Chunk::NV; ++u) {
-      kmax = at_absmax4(kc.v[u], kmax);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) vmax[e] = fmaxf(vmax[e], fabsf(vc.v[u][e]));
-    }
-  };
-  track();
-  float ik, iv, sk, sv;
-  {
-    float a = kmax, b = fmaxf(fmaxf(vmax[0], vmax[1]), fmaxf(vmax[2], vmax[3]));
-#pragma unroll
-    for (int x = 1; x < 64; x *= 2) {
-      a = fmaxf(a, __shfl_xor(a, x, 64));
-      b = fmaxf(b, __shfl_xor(b, x, 64));
-    }
-    if (lane == 0) {
-      red[wave] = a;
-      red[RB + wave] = b;
-    }
-    __syncthreads();
-    a = red[0];
-    b = red[RB];
-#pragma unroll
-    for (int x = 1; x < RB; ++x) {
-      a = fmaxf(a, red[x]);
-      b = fmaxf(b, red[RB + x]);
-    }
-    sk = at_pow2_scale(a, ik);
-    sv = at_pow2_scale(b, iv);
-  }
-  const float mult = p.scale2 * ik * iq;  // of a product of scaled rows
-  float m = 0.0f, l = 0.0f;               // reference score; sum of the weights
-  at_f16 o[ND], os[ND];                   // O^T: main and small products
-#pragma unroll
-  for (int nd = 0; nd < ND; ++nd) o[nd] = os[nd] = at_zero16();
-  auto stage = [&](int j) {
-    uint16_t* dst = Kt + (j & 1) * 4 * TS;
-    at_store_split<D, NT>(kc, sk, dst, j * kAtChunk, L);
-    at_store_split<D, NT>(vc, sv, dst + 2 * TS, j * kAtChunk, L);
-    kc.load(kp, p.st[kAtK][3], (j + 1) * kAtChunk, L);  // past L: row L - 1 again
-    vc.load(vp, p.st[kAtV][3], (j + 1) * kAtChunk, L);
-  };
-  stage(0);
-  __syncthreads();
-  // One chunk; `last` (a constant): the chunk with the keys past L, which stages nothing.
-  auto chunk = [&](auto last, int j) {
-    constexpr bool LAST = decltype(last)::value;
-    const uint16_t* Kj = Kt + (j & 1) * 4 * TS;
-    const uint16_t* Vj = Kj + 2 * TS;
-    at_f16 s0 = at_zero16(), s1 = at_zero16();  // the chunk's two key blocks
-    {
-      AtH8 a0[D / 16], a1[D / 16];
-#pragma unroll
-      for (int s = 0; s < D / 16; ++s) {
-        a0[s] = at_tile_row<D>(Kj, TS, col, 16 * s + 8 * grp);
-        a1[s] = at_tile_row<D>(Kj, TS, 32 + col, 16 * s + 8 * grp);
-      }
-#pragma unroll
-      for (int s = 0; s < D / 16; ++s) {  // small products first
-        at_mfma(s0, a0[s].h, qt[s].l);
-        at_mfma(s1, a1[s].h, qt[s].l);
-        at_mfma(s0, a0[s].l, qt[s].h);
-        at_mfma(s1, a1[s].l, qt[s].h);
-      }
-#pragma unroll
-      for (int s = 0; s < D / 16; ++s) {
-        at_mfma(s0, a0[s].h, qt[s].h);
-        at_mfma(s1, a1[s].h, qt[s].h);
-      }
-    }
-    if constexpr (!LAST) {
-      track();
-      stage(j + 1);
-      at_interleave<6 * D / 16, 10>();
-    }
-    float bm = -INFINITY;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      s0[i] = fmaf(s0[i], mult, -m);
-      s1[i] = fmaf(s1[i], mult, -m);
-      if (LAST) {
-        const int key = j * kAtChunk + 8 * (i >> 2) + 4 * grp + (i & 3);
-        s0[i] = key < L ? s0[i] : -INFINITY;
-        s1[i] = key + 32 < L ? s1[i] : -INFINITY;
-      }
-      bm = at_max3(bm, s0[i], s1[i]);
-    }
-    bm = at_max_halves(bm);  // relative to m; finite: every chunk holds a key below L
-    if (bm > 15.0f || (l == 0.0f && bm < 3.0f)) {
-      bm -= 7.0f;
-      const float alpha = l == 0.0f ? 0.0f : at_exp2(-bm);
-      m += bm;
-      l *= alpha;
-      s0 -= bm;
-      s1 -= bm;
-#pragma unroll
-      for (int nd = 0; nd < ND; ++nd) {
-        o[nd] *= alpha;
-        os[nd] *= alpha;
-      }
-    }
-    float rs = 0.0f;
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        at_f16& sc = h == 0 ? s0 : s1;
-#pragma unroll
-        for (int i = 8 * s; i < 8 * s + 8; ++i) {
-          sc[i] = at_exp2(sc[i]);
-          rs += sc[i];
-        }
-        const AtH8 b = at_split_regs(sc, 8 * s);
-#pragma unroll
-        for (int nd = 0; nd < ND; ++nd) {  // O^T += V^T P^T
-          const AtH8 a = at_tile_tr<D>(Vj, TS, 32 * h, nd, s, lane);
-          at_mfma(os[nd], a.h, b.l);
-          at_mfma(o[nd], a.h, b.h);
-          at_mfma(os[nd], a.l, b.h);
-        }
-      }
-    l += at_sum_halves(rs);
-  };
-  for (int j = 0; j + 1 < nchunks; ++j) {
-    if (qb < nb) {
-      chunk(std::false_type{}, j);
-    } else {
-      track();
-      stage(j + 1);
-    }
-    __syncthreads();  // chunk j + 1 is staged, and every wave is done with chunk j
-  }
-  if (qb < nb) chunk(std::true_type{}, nchunks - 1);
-  // Channels of V that the scale leaves too small: the largest element of each over the workgroup's
-  // threads (channels 4 c .. 4 c + 3 lie in threads c modulo D / 4)
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-#pragma unroll
-    for (int x = D / 4; x < 64; x *= 2) vmax[e] = fmaxf(vmax[e], __shfl_xor(vmax[e], x, 64));
-  }
-#pragma unroll
-  for (int x = 1; x < 64; x *= 2) kmax = fmaxf(kmax, __shfl_xor(kmax, x, 64));
-  if (lane < D / 4) *reinterpret_cast<at_f4*>(&red[wave * D + 4 * lane]) = vmax;
-  if (lane == 0) red[4 * D + wave] = kmax;
-  __syncthreads();
-#pragma unroll
-  for (int x = 0; x < RB; ++x) kmax = fmaxf(kmax, red[4 * D + x]);
-  bool bad = !(kmax * sk <= kAtF16Max) || (qv && !(qm * kmax * p.scale2 <= kAtMaxProduct));
-  if (static_cast<int>(threadIdx.x) < D) {
-    float v = 0.0f;
-#pragma unroll
-    for (int x = 0; x < RB; ++x) v = fmaxf(v, red[x * D + threadIdx.x]);
-    v *= sv;
-    bad = bad || !(v <= kAtF16Max) || (v != 0.0f && v < 0.5f);
-  }
-  const float inv = iv / l;
-  float z = 0.0f;  // NaN if a result is not finite
-#pragma unroll
-  for (int nd = 0; nd < ND; ++nd) {
-    o[nd] = (o[nd] + os[nd]) * inv;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) z = fmaf(o[nd][i], 0.0f, z);
-  }
-  if (__syncthreads_or(bad || (z != z && qv))) {
-    attn_fwd_body<float, D, false, RB, false>(p, w, at_lds);
-    return;
-  }
-  if (qb < nb) {
-    float* op = static_cast<float*>(p.out) + w.sl.base(p, kAtO);
-#pragma unroll
-    for (int nd = 0; nd < ND; ++nd) at_store_block<float>(op + 32 * nd, p.st[kAtO][3], qb * 32, L, o[nd], 1.0f, at_lds + wave * (at_scratch_bytes<float>() / 4), lane);
-    if (qv && grp == 0) {
-      float* stats = p.stats + (static_cast<int64_t>(w.zh) * L + qi) * 4;
-      // The weights sum to l = 2^e f, f in [1, 2): m + e, and log2 f with what m + e rounds off. The
-      // backward's s - stats[0] - stats[1] is then rounded at the size of the weight's own log2; with m
-      // and log2 l (3 to 24) the rounding of these was most of the gradients' error against float64:
-      // 300 x 32 4.3, 4.1, 4.2e-7 (grad_q, grad_k, grad_v) -> 2.3, 2.0, 1.9e-7; 50 x 32 3.0 -> 1.7e-7;
-      // 300 x 64 (backward on f32 MFMAs) 5.7, 6.0, 5.8e-7 -> 4.4, 4.7, 4.5e-7.
-      const float e = static_cast<float>(static_cast<int>(__float_as_uint(l) >> 23) - 127);
-      const float f = __uint_as_float((__float_as_uint(l) & 0x007fffffu) | 0x3f800000u);
-      const float me = m + e, t = me - m;
-      stats[0] = me;
-      stats[1] = log2f(f) + ((m - (me - t)) + (e - t));
-    }
-  }
-}
-
-// ---- backward: three bf16 terms ----------------------------------------------------------------
+// ---- operands of three bf16 terms --------------------------------------------------------------
 constexpr int kAtTerms = 3;
 
 // N f32 values (r, left as what the terms do not hold) as three bf16 terms packed in pairs, largest
@@ -462,6 +124,193 @@ __device__ __forceinline__ void at_operand_tr(at_bf8 (&a)[kAtTerms], const uint1
   for (int u = 0; u < kAtTerms; ++u) a[u] = at_bf8_of(at_read_tr(X + u * stride + at_swo<D>(ro, c)), at_read_tr(X + u * stride + at_swo<D>(ro + 8, c)));
 }
 
+// Asks the scheduler to follow each of the block's N MFMAs by up to V vector operations: it would
+// issue the dependent MFMAs back to back and the vector work after them.
+template <int N, int V>
+__device__ __forceinline__ void at_interleave() {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x2, V, 0);
+  }
+}
+
+// ---- forward ------------------------------------------------------------------------------------
+// Whether a non-zero |x| is below 2^-kAtLeastLog2, where the third term leaves bf16's range: the least of
+// (bits of x shifted past the sign) - 1, unsigned, over the values (a zero wraps to the largest).
+constexpr int kAtLeastLog2 = 100;
+__device__ __forceinline__ uint32_t at_least(const at_f4& v, uint32_t least) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) least = min(least, (__float_as_uint(v[e]) << 1) - 1u);
+  return least;
+}
+__device__ __forceinline__ bool at_too_small(uint32_t least) { return least < (static_cast<uint32_t>(127 - kAtLeastLog2) << 24) - 1u; }
+
+// An AtChunk (64 f32 rows in registers) as swizzled term tiles [term][64][D] (at_swo); rows past L are 0.
+template <int D, int NT>
+__device__ __forceinline__ void at_store_split(const AtChunk<float, D, NT>& ch, uint16_t* dst, int r0, int L) {
+#pragma unroll
+  for (int u = 0; u < AtChunk<float, D, NT>::NV; ++u) {
+    const int idx = threadIdx.x + NT * u, row = idx / (D / 4), c4 = idx - row * (D / 4);
+    uint2 t[kAtTerms];
+    at_split4(r0 + row < L ? ch.v[u] : at_f4{0.0f, 0.0f, 0.0f, 0.0f}, t);
+#pragma unroll
+    for (int q = 0; q < kAtTerms; ++q) *reinterpret_cast<uint2*>(&dst[q * kAtChunk * D + at_swo<D>(row, 4 * c4)]) = t[q];
+  }
+}
+
+// Key and value term tiles. head_dim 32 has two buffers (three workgroups a CU); two of head_dim 64 would leave one workgroup a CU.
+template <int D>
+constexpr int at_split_buffers() { return D == 32 ? 2 : 1; }
+template <int D>
+constexpr int at_split_lds_bytes() { return at_split_buffers<D>() * 2 * kAtTerms * kAtChunk * D * 2; }
+static_assert(at_split_lds_bytes<32>() >= at_lds_floats<32>() * 4 && at_split_lds_bytes<64>() >= at_lds_floats<64>() * 4, "the f32 body fits");
+
+// Forward (attn_fwd_kernel's work split and streaming). A workgroup splits each chunk once, at head_dim 32
+// into one of two buffers in the shadow of the chunk before's MFMAs. The softmax reference m is moved
+// when a chunk's largest weight would leave [2^3, 2^15] (the first chunk) or exceed 2^15.
+template <int D, int RB>
+__global__ void __launch_bounds__(64 * RB, D == 32 ? 3 : 2) attn_fwd_split_kernel(const AttnParams p) {
+  constexpr int NT = 64 * RB, ND = D / 32, TS = kAtChunk * D, NBUF = at_split_buffers<D>();  // TS: elements of a term tile
+  extern __shared__ __align__(16) float at_lds[];
+  uint16_t* Kt = reinterpret_cast<uint16_t*>(at_lds);  // [buffer][K, V][term][64][D]
+  const int L = p.len, nb = (L + 31) / 32, nchunks = (L + kAtChunk - 1) / kAtChunk;
+  const AttnWork w(p, (nb + RB - 1) / RB);
+  const float* kp = static_cast<const float*>(p.k) + w.sl.base(p, kAtK);
+  const float* vp = static_cast<const float*>(p.v) + w.sl.base(p, kAtV);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, grp = lane >> 5, col = lane & 31;
+  const int qb = w.rc * RB + wave, qi = qb * 32 + col;
+  const bool qv = qi < L;
+  using Chunk = AtChunk<float, D, NT>;
+  Chunk kc, vc;
+  kc.load(kp, p.st[kAtK][3], 0, L);
+  vc.load(vp, p.st[kAtV][3], 0, L);
+  uint32_t least = 0xffffffffu;
+  at_bf8 qt[D / 16][kAtTerms];
+  {
+    const float* qp = static_cast<const float*>(p.q) + w.sl.base(p, kAtQ) + at_row_off(min(qi, L - 1), p.st[kAtQ][3]);
+#pragma unroll
+    for (int s = 0; s < D / 16; ++s) {
+      const at_f4 a = *reinterpret_cast<const at_f4*>(qp + 16 * s + 8 * grp), b = *reinterpret_cast<const at_f4*>(qp + 16 * s + 8 * grp + 4);
+      least = at_least(b, at_least(a, least));
+      at_split8(at_f8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}, qt[s]);
+    }
+  }
+  float m = 0.0f, l = 0.0f;  // reference score; sum of the weights
+  at_f16 o[ND], os[ND];      // O^T: main and small products
+#pragma unroll
+  for (int nd = 0; nd < ND; ++nd) o[nd] = os[nd] = at_zero16();
+  auto stage = [&](int j) {
+    uint16_t* dst = Kt + (j % NBUF) * 2 * kAtTerms * TS;
+#pragma unroll
+    for (int u = 0; u < Chunk::NV; ++u) least = at_least(vc.v[u], at_least(kc.v[u], least));
+    at_store_split<D, NT>(kc, dst, j * kAtChunk, L);
+    at_store_split<D, NT>(vc, dst + kAtTerms * TS, j * kAtChunk, L);
+    kc.load(kp, p.st[kAtK][3], (j + 1) * kAtChunk, L);  // past L: row L - 1 again
+    vc.load(vp, p.st[kAtV][3], (j + 1) * kAtChunk, L);
+  };
+  stage(0);
+  __syncthreads();
+  // One chunk; `last` (a constant): the chunk with the keys past L, which stages nothing.
+  auto chunk = [&](auto last, int j) {
+    constexpr bool LAST = decltype(last)::value;
+    const uint16_t* Kj = Kt + (j % NBUF) * 2 * kAtTerms * TS;
+    const uint16_t* Vj = Kj + kAtTerms * TS;
+    at_f16 s0 = at_scores_split<D>(Kj, TS, 0, qt, col, grp), s1 = at_scores_split<D>(Kj, TS, 32, qt, col, grp);  // the chunk's two key blocks
+    if constexpr (!LAST && NBUF == 2) stage(j + 1);
+    float bm = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      s0[i] = fmaf(s0[i], p.scale2, -m);
+      s1[i] = fmaf(s1[i], p.scale2, -m);
+      if (LAST) {
+        const int key = j * kAtChunk + 8 * (i >> 2) + 4 * grp + (i & 3);
+        s0[i] = key < L ? s0[i] : -INFINITY;
+        s1[i] = key + 32 < L ? s1[i] : -INFINITY;
+      }
+      bm = at_max3(bm, s0[i], s1[i]);
+    }
+    bm = at_max_halves(bm);  // relative to m; finite: every chunk holds a key below L
+    if (bm > 15.0f || (l == 0.0f && bm < 3.0f)) {
+      bm -= 7.0f;
+      const float alpha = l == 0.0f ? 0.0f : at_exp2(-bm);
+      m += bm;
+      l *= alpha;
+      s0 -= bm;
+      s1 -= bm;
+#pragma unroll
+      for (int nd = 0; nd < ND; ++nd) {
+        o[nd] *= alpha;
+        os[nd] *= alpha;
+      }
+    }
+    float rs = 0.0f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        at_f16& sc = h == 0 ? s0 : s1;
+#pragma unroll
+        for (int i = 8 * s; i < 8 * s + 8; ++i) {
+          sc[i] = at_exp2(sc[i]);
+          rs += sc[i];
+        }
+        at_bf8 b[kAtTerms];
+        at_split_regs(sc, 8 * s, b);
+#pragma unroll
+        for (int nd = 0; nd < ND; ++nd) {  // O^T += V^T P^T
+          at_bf8 a[kAtTerms];
+          at_operand_tr<D>(a, Vj, TS, 32 * h, nd, s, lane);
+          at_mfma_small(os[nd], a, b);
+          at_mfma(o[nd], a[0], b[0]);
+        }
+      }
+    l += at_sum_halves(rs);
+  };
+  for (int j = 0; j + 1 < nchunks; ++j) {
+    if (qb < nb) chunk(std::false_type{}, j);
+    if constexpr (NBUF == 1) {
+      __syncthreads();  // every wave is done with chunk j
+      stage(j + 1);
+    } else if (qb >= nb) {
+      stage(j + 1);
+    }
+    __syncthreads();  // chunk j + 1 is staged, and every wave is done with chunk j
+  }
+  if (qb < nb) chunk(std::true_type{}, nchunks - 1);
+  const float inv = 1.0f / l;
+  float z = 0.0f;  // NaN if a result is not finite
+#pragma unroll
+  for (int nd = 0; nd < ND; ++nd) {
+    o[nd] = (o[nd] + os[nd]) * inv;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) z = fmaf(o[nd][i], 0.0f, z);
+  }
+  if (__syncthreads_or(at_too_small(least) || (z != z && qv))) {  // and every wave is done with the tiles
+    attn_fwd_body<float, D, false, RB, false>(p, w, at_lds);
+    return;
+  }
+  if (qb < nb) {
+    float* op = static_cast<float*>(p.out) + w.sl.base(p, kAtO);
+#pragma unroll
+    for (int nd = 0; nd < ND; ++nd) at_store_block<float>(op + 32 * nd, p.st[kAtO][3], qb * 32, L, o[nd], 1.0f, at_lds + wave * (at_scratch_bytes<float>() / 4), lane);
+    if (qv && grp == 0) {
+      float* stats = p.stats + (static_cast<int64_t>(w.zh) * L + qi) * 4;
+      // The weights sum to l = 2^e f, f in [1, 2): m + e, and log2 f with what m + e rounds off. The
+      // backward's s - stats[0] - stats[1] is then rounded at the size of the weight's own log2; with m
+      // and log2 l (3 to 24) the rounding of these was most of the gradients' error against float64:
+      // 300 x 32 4.3, 4.1, 4.2e-7 (grad_q, grad_k, grad_v) -> 2.3, 2.0, 1.9e-7; 50 x 32 3.0 -> 1.7e-7;
+      // 300 x 64 (backward on f32 MFMAs) 5.7, 6.0, 5.8e-7 -> 4.4, 4.7, 4.5e-7.
+      const float e = static_cast<float>(static_cast<int>(__float_as_uint(l) >> 23) - 127);
+      const float f = __uint_as_float((__float_as_uint(l) & 0x007fffffu) | 0x3f800000u);
+      const float me = m + e, t = me - m;
+      stats[0] = me;
+      stats[1] = log2f(f) + ((m - (me - t)) + (e - t));
+    }
+  }
+}
+
+// ---- fused backward -----------------------------------------------------------------------------
 // Fused backward: one workgroup per (slice, head), one phase per 32-row query block. Key waves (one
 // per key block, K and V terms in registers) form S, dP, P and dS of their block against the
 // phase's query block, write dS as three term tiles [32 keys][32 queries], and accumulate dV and dK.

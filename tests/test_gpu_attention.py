@@ -692,3 +692,72 @@ def test_split_forward_statistics(shape):
     want = x.max(-1) + np.log2(np.exp2(x - x.max(-1, keepdims=True)).sum(-1))
     assert np.abs(st[..., 0] + st[..., 1] - want).max() <= 5.6e-6
     assert st[..., 1].min() >= -(2.0 ** -20) and st[..., 1].max() <= 1.0 + 2.0 ** -20
+
+
+def _row_range_inputs(kind, shape):
+    """Keys, values and queries whose rows differ so much in size that a scale shared by rows, or taken from
+    the first of them, would cost some rows their low bits."""
+    rng = np.random.default_rng(63)
+    q, k, v = (rng.standard_normal(shape).astype(np.float32) for _ in range(3))
+    if kind.startswith("zero_first"):  # nothing in the first chunk; scores of ordinary size from small keys
+        size = np.float32(kind[len("zero_first_"):])
+        k[:, :, :64] = 0.0
+        q, k = q / size, k * size
+    elif kind.startswith("large_row"):  # one value row far above the others, which no query attends to
+        q[..., 0], k[:, :, 5, 0] = 3.0, -250.0
+        v[:, :, 5] *= np.float32(kind[len("large_row_"):])
+    elif kind == "value_rows":  # every query attends to its own key; values from 1e-8 to 1
+        k = (k / np.linalg.norm(k, axis=-1, keepdims=True) * 12.0).astype(np.float32)
+        q = k * np.float32(np.sqrt(shape[-1]) / 3.0)
+        v = (v * 10.0 ** rng.uniform(-8, 0, (*shape[:3], 1))).astype(np.float32)
+    else:  # keys from 1e-8 to 1
+        k = (k * 10.0 ** rng.uniform(-8, 0, (*shape[:3], 1))).astype(np.float32)
+    return q, k, v
+
+
+ROW_RANGES = ["zero_first_1e-4", "zero_first_1e-6", "zero_first_1e4", "large_row_1e6", "large_row_1e8", "value_rows", "key_rows"]
+
+
+@pytest.mark.parametrize("kind", ROW_RANGES)
+@pytest.mark.parametrize("shape", [(2, 2, 300, 32), (1, 3, 130, 64)], ids=str)
+def test_split_forward_keeps_every_row(shape, kind):
+    """The maskless f32 forward (split operands) against the f32 matrix kernel (a mask that blocks nothing),
+    row by row: the largest error of a query's output row, relative to the row's sum of weights times |values|,
+    and of the statistics, is at most twice that kernel's and a rounding of f32 (2^-23; the statistics' log2
+    of a sum near 2^8 is rounded at 2^-20)."""
+    from rfdetr_jax_amd.attention import _Layout, attention_forward
+
+    _note(f"split forward rows {kind} {shape}")
+    q, k, v = _row_range_inputs(kind, shape)
+    b, h, length, d = shape
+    lay = _Layout(b, 1, h, length, d)
+    x = np.matmul(q.astype(np.float64), k.astype(np.float64).swapaxes(-1, -2)) / np.sqrt(d)
+    top = x.max(-1, keepdims=True)
+    weights = np.exp(x - top)
+    total = weights.sum(-1, keepdims=True)
+    weights /= total
+    want, size = weights @ v.astype(np.float64), weights @ np.abs(v.astype(np.float64))
+    log2_sum = ((top + np.log(total)) * np.log2(np.e))[..., 0]
+    errors = []
+    for mask in (None, _t(np.zeros((length, length), bool))):
+        out, stats = attention_forward(_t(q), _t(k), _t(v), lay, lay.strides_bhld, mask)
+        torch.cuda.synchronize()
+        st = _np(stats).reshape(b, h, length, 4).astype(np.float64)
+        rows = np.linalg.norm(_np(out).astype(np.float64) - want, axis=-1) / np.linalg.norm(size, axis=-1)
+        errors.append((rows.max(), np.abs(st[..., 0] + st[..., 1] - log2_sum).max()))
+    (out_split, st_split), (out_f32, st_f32) = errors
+    _note(f"rows: {out_split:.2g} against {out_f32:.2g}; statistics: {st_split:.2g} against {st_f32:.2g}")
+    assert out_split <= 2 * out_f32 + 2.0 ** -23
+    assert st_split <= 2 * st_f32 + 2.0 ** -20
+
+
+@pytest.mark.parametrize("d", [32, 64])
+def test_split_forward_of_one_key_returns_the_value(d):
+    """With one key the weight is 1 and every bit of the value comes back, as from the f32 kernel."""
+    rng = np.random.default_rng(64)
+    q, k = (_t(rng.standard_normal((4, 8, 1, d)).astype(np.float32)) for _ in range(2))
+    v = _t((rng.standard_normal((4, 8, 1, d)) * 10.0 ** rng.uniform(-9, 9, (4, 8, 1, d))).astype(np.float32))
+    q[0] = 0.0  # a score of exactly 0, the others' weight is 2^x for a rounded x: f32's rounding of w v / w
+    out = scaled_dot_product_attention(q, k, v)
+    assert torch.equal(out[0], v[0])
+    assert float(((out - v).abs() / v.abs()).max()) <= 2.0 ** -22
