@@ -9,8 +9,8 @@
 // left out is below 2^-25 of a product, under the rounding of an f32 product. bf16 products run at 16
 // times the rate of f32 ones (10 times measured: dense bf16 MFMAs reach 1.6 PFLOP/s here); sums are f32.
 // A workgroup whose results are not all finite (an infinity, or a value that rounds to one in bf16,
-// leaves the split as NaN), and in the forward one that meets a non-zero element below 2^-100, does its
-// work again in the f32 kernel's body. Such a workgroup takes the time of both.
+// leaves the split as NaN), or that meets a non-zero element of its inputs below 2^-100, does its work
+// again in the f32 kernel's body. Such a workgroup takes the time of both.
 // (Two f16 terms, scaled into f16's range, took 62 us where three bf16 terms take 84, and lost bits: the
 // low ones of a quarter of all values, and of rows far below the size that the scale was taken from,
 // with relative errors of 1e-2 at a spread of 1e8.)
@@ -73,13 +73,33 @@ __device__ __forceinline__ void at_split_regs(const at_f16& v, int i0, at_bf8 (&
   at_split8(at_f8{v[i0], v[i0 + 1], v[i0 + 2], v[i0 + 3], v[i0 + 4], v[i0 + 5], v[i0 + 6], v[i0 + 7]}, t);
 }
 
+// Whether a non-zero element is below 2^-100, where the third term leaves bf16's range, by the first terms
+// (packed pairs): the least of (16 bits shifted past the sign) - 1, unsigned, so that 0 wraps to the
+// largest. One multiply-add and one minimum a pair; on the f32 values, which takes three operations a
+// pair, the backward's dQ waves made it 231 us where this way and no check are both 222.
+typedef uint16_t at_u2 __attribute__((ext_vector_type(2)));
+constexpr int kAtLeastLog2 = 100;
+__device__ __forceinline__ void at_least(at_u2& least, uint32_t pair) {
+  least = __builtin_elementwise_min(least, __builtin_bit_cast(at_u2, pair) * static_cast<uint16_t>(2) - static_cast<uint16_t>(1));
+}
+__device__ __forceinline__ void at_least(at_u2& least, const at_bf8& t) {
+  const uint4 w = __builtin_bit_cast(uint4, t);
+  at_least(least, w.x);
+  at_least(least, w.y);
+  at_least(least, w.z);
+  at_least(least, w.w);
+}
+__device__ __forceinline__ bool at_too_small(const at_u2& least) { return min(least.x, least.y) < (127 - kAtLeastLog2) * 256; }
+constexpr at_u2 kAtNoneSmall = {0xffff, 0xffff};
+
 // channels 16 s + 8 grp .. + 7 of a 16-byte aligned f32 row, s < D / 16
 template <int D>
-__device__ __forceinline__ void at_row_split(at_bf8 (&t)[D / 16][kAtTerms], const float* row, int grp) {
+__device__ __forceinline__ void at_row_split(at_bf8 (&t)[D / 16][kAtTerms], const float* row, int grp, at_u2& least) {
 #pragma unroll
   for (int s = 0; s < D / 16; ++s) {
     const at_f4 a = *reinterpret_cast<const at_f4*>(row + 16 * s + 8 * grp), b = *reinterpret_cast<const at_f4*>(row + 16 * s + 8 * grp + 4);
     at_split8(at_f8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}, t[s]);
+    at_least(least, t[s][0]);
   }
 }
 
@@ -136,24 +156,16 @@ __device__ __forceinline__ void at_interleave() {
 }
 
 // ---- forward ------------------------------------------------------------------------------------
-// Whether a non-zero |x| is below 2^-kAtLeastLog2, where the third term leaves bf16's range: the least of
-// (bits of x shifted past the sign) - 1, unsigned, over the values (a zero wraps to the largest).
-constexpr int kAtLeastLog2 = 100;
-__device__ __forceinline__ uint32_t at_least(const at_f4& v, uint32_t least) {
-#pragma unroll
-  for (int e = 0; e < 4; ++e) least = min(least, (__float_as_uint(v[e]) << 1) - 1u);
-  return least;
-}
-__device__ __forceinline__ bool at_too_small(uint32_t least) { return least < (static_cast<uint32_t>(127 - kAtLeastLog2) << 24) - 1u; }
-
 // An AtChunk (64 f32 rows in registers) as swizzled term tiles [term][64][D] (at_swo); rows past L are 0.
 template <int D, int NT>
-__device__ __forceinline__ void at_store_split(const AtChunk<float, D, NT>& ch, uint16_t* dst, int r0, int L) {
+__device__ __forceinline__ void at_store_split(const AtChunk<float, D, NT>& ch, uint16_t* dst, int r0, int L, at_u2& least) {
 #pragma unroll
   for (int u = 0; u < AtChunk<float, D, NT>::NV; ++u) {
     const int idx = threadIdx.x + NT * u, row = idx / (D / 4), c4 = idx - row * (D / 4);
     uint2 t[kAtTerms];
     at_split4(r0 + row < L ? ch.v[u] : at_f4{0.0f, 0.0f, 0.0f, 0.0f}, t);
+    at_least(least, t[0].x);
+    at_least(least, t[0].y);
 #pragma unroll
     for (int q = 0; q < kAtTerms; ++q) *reinterpret_cast<uint2*>(&dst[q * kAtChunk * D + at_swo<D>(row, 4 * c4)]) = t[q];
   }
@@ -185,16 +197,11 @@ __global__ void __launch_bounds__(64 * RB, D == 32 ? 3 : 2) attn_fwd_split_kerne
   Chunk kc, vc;
   kc.load(kp, p.st[kAtK][3], 0, L);
   vc.load(vp, p.st[kAtV][3], 0, L);
-  uint32_t least = 0xffffffffu;
+  at_u2 least = kAtNoneSmall;
   at_bf8 qt[D / 16][kAtTerms];
   {
     const float* qp = static_cast<const float*>(p.q) + w.sl.base(p, kAtQ) + at_row_off(min(qi, L - 1), p.st[kAtQ][3]);
-#pragma unroll
-    for (int s = 0; s < D / 16; ++s) {
-      const at_f4 a = *reinterpret_cast<const at_f4*>(qp + 16 * s + 8 * grp), b = *reinterpret_cast<const at_f4*>(qp + 16 * s + 8 * grp + 4);
-      least = at_least(b, at_least(a, least));
-      at_split8(at_f8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}, qt[s]);
-    }
+    at_row_split<D>(qt, qp, grp, least);
   }
   float m = 0.0f, l = 0.0f;  // reference score; sum of the weights
   at_f16 o[ND], os[ND];      // O^T: main and small products
@@ -202,10 +209,8 @@ __global__ void __launch_bounds__(64 * RB, D == 32 ? 3 : 2) attn_fwd_split_kerne
   for (int nd = 0; nd < ND; ++nd) o[nd] = os[nd] = at_zero16();
   auto stage = [&](int j) {
     uint16_t* dst = Kt + (j % NBUF) * 2 * kAtTerms * TS;
-#pragma unroll
-    for (int u = 0; u < Chunk::NV; ++u) least = at_least(vc.v[u], at_least(kc.v[u], least));
-    at_store_split<D, NT>(kc, dst, j * kAtChunk, L);
-    at_store_split<D, NT>(vc, dst + kAtTerms * TS, j * kAtChunk, L);
+    at_store_split<D, NT>(kc, dst, j * kAtChunk, L, least);
+    at_store_split<D, NT>(vc, dst + kAtTerms * TS, j * kAtChunk, L, least);
     kc.load(kp, p.st[kAtK][3], (j + 1) * kAtChunk, L);  // past L: row L - 1 again
     vc.load(vp, p.st[kAtV][3], (j + 1) * kAtChunk, L);
   };
@@ -352,6 +357,7 @@ __global__ void __launch_bounds__(64 * (kAtFusedBlocks + 2), 3) attn_bwd_fused_s
   if (wave < nb) {  // key block kb = wave (uniform per wave)
     const int kb = wave, kcl = min(kb * 32 + col, L - 1);
     at_bf8 kt[D / 16][kAtTerms], vt[D / 16][kAtTerms];
+    at_u2 least = kAtNoneSmall;
     {
       at_f4 kc[4];  // the block's rows of the key copy: row 8 u + lane / 8, channels 4 (lane % 8) .. + 3
 #pragma unroll
@@ -359,8 +365,8 @@ __global__ void __launch_bounds__(64 * (kAtFusedBlocks + 2), 3) attn_bwd_fused_s
         const int row = kb * 32 + 8 * u + (lane >> 3);
         kc[u] = row < L ? *reinterpret_cast<const at_f4*>(kp + at_row_off(row, p.st[kAtK][3]) + 4 * (lane & 7)) : at_f4{0.0f, 0.0f, 0.0f, 0.0f};
       }
-      at_row_split<D>(kt, kp + at_row_off(kcl, p.st[kAtK][3]), grp);
-      at_row_split<D>(vt, static_cast<const float*>(p.v) + sl.base(p, kAtV) + at_row_off(kcl, p.st[kAtV][3]), grp);
+      at_row_split<D>(kt, kp + at_row_off(kcl, p.st[kAtK][3]), grp, least);
+      at_row_split<D>(vt, static_cast<const float*>(p.v) + sl.base(p, kAtV) + at_row_off(kcl, p.st[kAtV][3]), grp, least);
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         uint2 x[kAtTerms];
@@ -370,7 +376,8 @@ __global__ void __launch_bounds__(64 * (kAtFusedBlocks + 2), 3) attn_bwd_fused_s
       }
     }
     at_f16 dk = at_zero16(), dv = at_zero16();
-    __syncthreads();  // query block 0 staged, key terms written
+    __syncthreads();  // query block 0 staged, key terms written, the flag cleared
+    if (at_too_small(least)) *bad = 1;
     for (int j = 0, b = 0; j < nb; ++j, b = b == 2 ? 0 : b + 1) {
       const uint16_t* Qb = Qt + b * kAtTerms * TR;
       const uint16_t* Gb = Gt + b * kAtTerms * TR;
@@ -460,6 +467,7 @@ __global__ void __launch_bounds__(64 * (kAtFusedBlocks + 2), 3) attn_bwd_fused_s
     const int srow = tq >> 2, sq4 = tq & 3;
     at_f8 qv, gv, ov;
     float2 sq = {0.0f, 0.0f};  // m, log2 l
+    at_u2 least = kAtNoneSmall;
     auto ld8 = [](const float* e) {
       const at_f4 a = *reinterpret_cast<const at_f4*>(e), b = *reinterpret_cast<const at_f4*>(e + 4);
       return at_f8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
@@ -485,6 +493,8 @@ __global__ void __launch_bounds__(64 * (kAtFusedBlocks + 2), 3) attn_bwd_fused_s
         *reinterpret_cast<uint4*>(&Qt[(b * kAtTerms + u) * TR + at_swo<D>(srow, 8 * sq4)]) = __builtin_bit_cast(uint4, qs[u]);
         *reinterpret_cast<uint4*>(&Gt[(b * kAtTerms + u) * TR + at_swo<D>(srow, 8 * sq4)]) = __builtin_bit_cast(uint4, gs[u]);
       }
+      at_least(least, qs[0]);
+      at_least(least, gs[0]);
       // the row's four quarters: neighbouring lanes (DPP quad_perm [1, 0, 3, 2], then [2, 3, 0, 1])
       dd += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(dd), 0xB1, 0xF, 0xF, false));
       dd += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(dd), 0x4E, 0xF, 0xF, false));
@@ -556,7 +566,7 @@ __global__ void __launch_bounds__(64 * (kAtFusedBlocks + 2), 3) attn_bwd_fused_s
       __syncthreads();
     }
     dq(nb - 1);
-    if (z != z) *bad = 1;
+    if (z != z || at_too_small(least)) *bad = 1;
     __syncthreads();
   }
   if (*bad != 0) {  // the same for every thread: read after the last barrier

@@ -761,3 +761,28 @@ def test_split_forward_of_one_key_returns_the_value(d):
     out = scaled_dot_product_attention(q, k, v)
     assert torch.equal(out[0], v[0])
     assert float(((out - v).abs() / v.abs()).max()) <= 2.0 ** -22
+
+
+@pytest.mark.parametrize("where", ["g", "v", "k", "q"])
+@pytest.mark.parametrize("length", [300, 33])
+def test_split_backward_of_tiny_tensors(tune, where, length):
+    """Elements of 1e-34, whose low bits leave bf16's range, cost the fused backward no bits: its gradients'
+    errors against float64 are at most twice the two-kernel f32 backward's (and 2^-23)."""
+    rng = np.random.default_rng(65)
+    shape = (2, 2, length, 32)
+    x = {n: rng.standard_normal(shape).astype(np.float32) for n in "qkvg"}
+    x[where] *= np.float32(1e-34)
+    if where in "qk":  # gradients within f32's range
+        x["g"] *= np.float32(1e10)
+        x["q" if where == "k" else "k"] *= np.float32(1e10)
+    want = AT.sdpa_vjp(x["q"], x["k"], x["v"], x["g"])
+    errors = []
+    for fused in (1, 0):
+        tune({"MSDA_ATTN_FUSED": fused})
+        t = [_t(x[n]).requires_grad_(True) for n in "qkv"]
+        got = torch.autograd.grad(scaled_dot_product_attention(*t), t, _t(x["g"]))
+        torch.cuda.synchronize()
+        errors.append([np.linalg.norm(_np(a).astype(np.float64) - b) / np.linalg.norm(b) for a, b in zip(got, want)])
+    _note(f"tiny {where} {length}: {errors}")
+    for name, split, f32 in zip("qkv", *errors):
+        assert split <= 2 * f32 + 2.0 ** -23, name
