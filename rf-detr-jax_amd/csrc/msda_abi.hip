@@ -507,13 +507,17 @@ int plan_band(const Shape& s, int vbytes, int ch, const DevInfo& dev, BandPlan* 
       // longer than a CU's share of all items, it gets one more band. In points: an item costs the
       // points of rows + 1 of its level's h rows, and 5.5 us, which is 300 points of 32 channels
       // (18 ns each). f32, 8 heads of 32, 900 queries x 4 points: eight images of 30x40 + 15x20
-      // levels, the coarse one a single item: backward 80 us without this rule and 71 with it; two
-      // images of 64x85, 32x43, 16x22, 8x11: 79 and 76; eight of them, with items to spare, are as before.
+      // levels, the coarse one a single item: core backward 65 us without this rule and 56 with it; two
+      // images of 64x85, 32x43, 16x22, 8x11: 66 and 58; eight of them, with items to spare, are as before.
+      // But no band that starts another round of a workgroup per CU: with a round's items exactly (often
+      // what the loop above leaves) one more a slice is a second round, 16 heads of 16, 500 queries, f32: four
+      // images of 30x29 + 15x14 19 us without and 28 with it, one of 53x37 + 26x18 14 and 23 (bf16).
       const double fixed = 300.0 * 32 / s.dim, all = static_cast<double>(s.queries) * s.points;
       auto cost = [&](int l) {
         const int rows = (s.h[l] + bp->bands[l] - 1) / bp->bands[l];
         return fixed + all * std::min(rows + 1, s.h[l]) / s.h[l];
       };
+      const auto rounds = [&](int64_t bands) { return (N * bands + target - 1) / target; };
       for (;;) {
         int top = 0;
         double sum = 0.0;
@@ -522,8 +526,10 @@ int plan_band(const Shape& s, int vbytes, int ch, const DevInfo& dev, BandPlan* 
           if (cost(l) > cost(top)) top = l;
         }
         const double longest = cost(top);
-        if (bp->bands[top] >= s.h[top] || longest * static_cast<double>(target) <= static_cast<double>(N) * sum) break;
+        if (bp->bands[top] >= s.h[top] || longest * static_cast<double>(target) <= static_cast<double>(N) * sum || rounds(nb_total + 1) > rounds(nb_total))
+          break;
         ++bp->bands[top];
+        ++nb_total;
       }
     }
   }
