@@ -57,6 +57,7 @@ struct BandParams {
   int heads, dim, queries, levels, points;
   int64_t len_value;
   int nwork;       // (level, band) items per slice
+  int run;         // slices whose items are taken together
   int nqb;         // query blocks per (slice, item); with part, each block writes a partial sum
   int qblock;      // queries per block
   float* part;     // nqb > 1 and grad_value requested: partial grad_value sums [nqb][B*H][S][D] (f32),
@@ -346,15 +347,16 @@ __global__ void __launch_bounds__(kBandMaxThreads) bwd_band_kernel(const BandPar
   extern __shared__ __align__(16) unsigned char lds_raw[];
   const int nt = blockDim.x, tid = threadIdx.x;
   const int lid = xcd_logical(blockIdx.x, gridDim.x);
-  // batch-major logical order: the workgroups of one batch entry (which share its location,
-  // weight and grad_output rows) run on one XCD
-  const int per_b = p.heads * p.nwork * p.nqb;
-  const int b = lid / per_b;
-  int rest = lid - b * per_b;
-  const int item = rest / (p.heads * p.nqb);
-  rest -= item * p.heads * p.nqb;
-  const int qb = rest / p.heads;
-  const int h = rest - qb * p.heads;
+  // Logical order: runs of `run` slices (b, h), a run's items by falling length, its query blocks, its
+  // slices.
+  const int per_run = p.run * p.nwork * p.nqb;
+  const int run_id = lid / per_run;
+  int rest = lid - run_id * per_run;
+  const int item = rest / (p.run * p.nqb);
+  rest -= item * p.run * p.nqb;
+  const int qb = p.nqb > 1 ? rest / p.run : 0;
+  const int pair = run_id * p.run + rest - qb * p.run;
+  const int b = pair / p.heads, h = pair - b * p.heads;
   const BandItem bi = band_item(p, item);
   const LevelDesc L = p.lv[bi.l];
   const int W = L.w, D = KD > 0 ? KD : p.dim, Q = p.queries, P = p.points, LP = p.levels * p.points;

@@ -507,3 +507,18 @@ def test_far_out_locations_contribute_nothing():
     assert_close(ga, ra, 1e-4, "grad_attn")
     ga5 = ga.reshape(loc.shape[:-1])
     assert not ga5[sel].any() and not gl[sel].any()
+
+
+@pytest.mark.parametrize("batch, heads", [(1, 8), (3, 8), (2, 4), (5, 3), (9, 8), (16, 4), (1, 16), (12, 2)])
+def test_band_backward_order_of_slices(batch, heads):
+    """Banded levels with the slices taken by batch entry (a batch of 8, or slices that do not divide by 8) and
+    by an XCD's share of them, several query passes' worth of points per level."""
+    shapes = ((33, 40), (9, 7), (17, 20))
+    _note(f"band order b{batch} h{heads}")
+    value, loc, attn, grad = make_inputs(70 + batch, batch, heads, 32, 90, shapes, 3, uniform_locations=True)
+    out, (gv, gl, ga) = _run(value, shapes, loc, attn, grad)
+    rv, rl, ra = R.ms_deform_attn_core_rows_vjp(value, shapes, loc, attn, grad)
+    assert_close(out, R.ms_deform_attn_core_rows(value, shapes, loc, attn), 1e-5, "out")
+    assert_close(gv, rv, 1e-4, "grad_value")
+    assert_close(gl, rl, 1e-4, "grad_loc")
+    assert_close(ga, ra, 1e-4, "grad_attn")
