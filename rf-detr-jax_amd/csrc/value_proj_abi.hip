@@ -112,10 +112,15 @@ int launch_gw(const msda::ValueProjParams& p, hipStream_t st) {
 //   * Rows: two column blocks a workgroup where that leaves four waves (32-row tiles) a CU, else one:
 //     bf16 8 x 576 rows forward 6.4 (one) against 6.6 us, 16 x 6800 42 against 33; four and eight
 //     blocks were slower at every size (52 and 55 us), their LDS leaving room for 8 waves a CU.
-//     f32 takes the path from four waves a CU on: at 1152 rows gemm4_kernel takes 6.5 us against 9.4,
-//     at 4608 13.6 against 13.5 (grad_input 14.1 against 12.0), at 16416 32.9 against 24.3.
-//   * grad_weight: 128-wide tiles (bf16) where they make one workgroup a CU; f32 from 16 slices (4096
-//     rows) on: at 1152 rows 11.8 us against 15.4, at 4608 20.0 against 18.4.
+//     f32 (256 -> 256, forward): two blocks with more than four waves a CU (8192 rows, four: 18.1, one block
+//     15.4; 9216: 18.3 and 21.9, gemm4_kernel 20.3), else one from four waves a CU on. From more than six it is
+//     the faster kernel (6800 rows 15.0 and 17.3), from four to six the closer one to float64 (7e-8 and
+//     1.1e-7; 4608 rows 14.6 and 13.6, grad_input 14.7 and 14.1; 128 columns, 9216 rows 10.7 and 9.3).
+//   * grad_weight: 128-wide tiles (bf16) where they make one workgroup a CU. f32 from 16 slices (4096
+//     rows) on (1152 rows 11.8 us by gemm4_kernel, 15.4), with workgroups for 5 of 8 CUs (64 x 64, one tile
+//     and 64 slices, at 108800 rows 42 and 56; 128 x 128 at 8192 rows, half the CUs, 12.7 and 14.6; at 16416,
+//     all of them, 21.2 and 20.0; 512 x 64 at 16416, two for each, 33 and 23; 160 x 160 at 4096, 9 of 16, 12.0
+//     and 14.0; 256 x 256 at 4608, 20.3 and 17.3).
 // MSDA_VP_CB=1 or 2 forces the path and the column blocks.
 template <int KIND, typename VT>
 int launch_mfma(const msda::ValueProjParams& p, hipStream_t st) {
@@ -128,16 +133,18 @@ int launch_mfma(const msda::ValueProjParams& p, hipStream_t st) {
     if constexpr (bf) {
       const int64_t t128 = static_cast<int64_t>((p.n + 127) / 128) * ((p.k + 127) / 128) * p.splits;
       if (t128 >= cus) return p.mask != nullptr ? launch_gw<VT, 128, true>(p, st) : launch_gw<VT, 128, false>(p, st);
-    } else if (p.splits < 16 && cb == 0) {
-      return MSDA_ERR_UNSUPPORTED;
+    } else if (cb == 0) {
+      const int64_t tiles = static_cast<int64_t>((p.n + 63) / 64) * ((p.k + 63) / 64);
+      if (p.splits < 16 || 8 * tiles * p.splits < 5 * int64_t{cus}) return MSDA_ERR_UNSUPPORTED;
     }
     return p.mask != nullptr ? launch_gw<VT, 64, true>(p, st) : launch_gw<VT, 64, false>(p, st);
   } else {
     const int cols = KIND == msda::kGemmForward ? p.n : p.k, red = KIND == msda::kGemmForward ? p.k : p.n;
     const int64_t tiles = (static_cast<int64_t>(p.batch) * p.seq + 31) / 32;
-    if (msda::VpRows<KIND, VT, 2>::lds_bytes(red) <= lds && (cb ? cb == 2 : tiles * ((cols + 63) / 64) >= 4 * int64_t{cus}))
+    const int64_t two = tiles * ((cols + 63) / 64), one = tiles * ((cols + 31) / 32);  // waves
+    if (msda::VpRows<KIND, VT, 2>::lds_bytes(red) <= lds && (cb ? cb == 2 : bf ? two >= 4 * int64_t{cus} : two > 4 * int64_t{cus}))
       return launch_rows<KIND, VT, 2>(p, lds, cus, st);
-    if (msda::VpRows<KIND, VT, 1>::lds_bytes(red) <= lds && (cb ? cb == 1 : bf || tiles * ((cols + 31) / 32) >= 4 * int64_t{cus}))
+    if (msda::VpRows<KIND, VT, 1>::lds_bytes(red) <= lds && (cb ? cb == 1 : bf || one >= 4 * int64_t{cus}))
       return launch_rows<KIND, VT, 1>(p, lds, cus, st);
     return MSDA_ERR_UNSUPPORTED;
   }
