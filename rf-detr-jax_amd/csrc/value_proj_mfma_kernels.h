@@ -10,7 +10,10 @@
 // 16 rows (v_mfma_f32_32x32x2_f32 in brackets): output 7e-8 (1.1e-7), grad_input 9e-8 (1.5e-7),
 // grad_weight 1.1e-7 to 2.5e-7 (1.6e-7 to 3.9e-7). The split turns an infinity (or a value that
 // rounds to one in bf16) into NaN, so a wave whose sums are not all finite computes its block again
-// in plain f32.
+// in plain f32, runs of 8 columns and indices at a time: with an infinity in one row the 4608-row forward
+// takes 61 us instead of 17, grad_weight 45 instead of 19, at 108800 rows 235 (94) and 397 (124), with one in
+// the weights, which every row meets, 88 and 1200. (One product at a time took 393 and 540 us, 893 and 3750,
+// 947 and 13300.)
 //
 // Measured (graph replays, 256 -> 16 x 16, us; v_mfma_f32 kernels before -> these):
 //   bf16 16 x 6800 rows: forward 207 -> 34, grad_input 221 -> 31, grad_weight and bias 219 -> 44
@@ -286,29 +289,44 @@ __global__ void __launch_bounds__((VpRows<KIND, VT, CB>::kThreads)) vp_rows_kern
   };
   // column (from c0) of register i of block j
   auto col = [&](int j, int i) { return 32 * j + 16 * (i >> 3) + 8 * half + (i & 7); };
+  // The tile's sums as plain f32 products, eight reduction indices at a time.
+  auto redo = [&](int mc) {
+    const uint32_t row = KIND == kGemmForward ? static_cast<uint32_t>(mc) * static_cast<uint32_t>(K) : vp_row_part(p, mc);
+#pragma unroll
+    for (int j = 0; j < CB; ++j) acc[j].clear();
+#pragma unroll 1
+    for (int r = 0; r < 8 * rc; r += 8) {
+      const vp_f4* src = reinterpret_cast<const vp_f4*>(static_cast<const float*>(act) + row +
+                                                        (KIND == kGemmForward ? static_cast<uint32_t>(r) : vp_col_part(p, r)));
+      const vp_f4 x[2] = {src[0], src[1]};
+#pragma unroll
+      for (int j = 0; j < CB; ++j)
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          const uint32_t c = static_cast<uint32_t>(min(c0 + col(j, 8 * g), C - 8));  // a run of 8 columns
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            // forward: column c + i at the eight indices; grad_input: the eight columns at index r + i
+            const uint32_t at = KIND == kGemmForward ? (c + static_cast<uint32_t>(i)) * static_cast<uint32_t>(K) + static_cast<uint32_t>(r)
+                                                     : static_cast<uint32_t>(r + i) * static_cast<uint32_t>(K) + c;
+            const vp_f4* w = reinterpret_cast<const vp_f4*>(p.w + at);
+            const vp_f4 lo = w[0], hi = w[1];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+              const float wq = q < 4 ? lo[q & 3] : hi[q & 3];
+              if (KIND == kGemmForward) acc[j].main[8 * g + i] = fmaf(x[q >> 2][q & 3], wq, acc[j].main[8 * g + i]);
+              else acc[j].main[8 * g + q] = fmaf(x[i >> 2][i & 3], wq, acc[j].main[8 * g + q]);
+            }
+          }
+        }
+    }
+  };
   auto finish = [&](int tl, bool padded) {
     asm volatile("" ::: "memory");  // keeps the bias reads here: hoisted out of the loop they take 16 CB registers
     const int m = tl * 32 + (lane & 31);
     const int mc = min(m, M - 1);
     if constexpr (!bf) {
-      if (vp_any_nonfinite(acc, padded || m >= M)) {
-        const uint32_t row = KIND == kGemmForward ? static_cast<uint32_t>(mc) * static_cast<uint32_t>(K) : vp_row_part(p, mc);
-#pragma unroll
-        for (int j = 0; j < CB; ++j)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int c = min(c0 + col(j, i), C - 1);
-            float s = 0.0f;
-            for (int r = 0; r < 8 * rc; ++r) {
-              const float x = static_cast<const float*>(act)[row + (KIND == kGemmForward ? static_cast<uint32_t>(r) : vp_col_part(p, r))];
-              const float w = KIND == kGemmForward ? p.w[static_cast<uint32_t>(c) * static_cast<uint32_t>(K) + static_cast<uint32_t>(r)]
-                                                   : p.w[static_cast<uint32_t>(r) * static_cast<uint32_t>(K) + static_cast<uint32_t>(c)];
-              s = fmaf(x, w, s);
-            }
-            acc[j].main[i] = s;
-            acc[j].small[i] = 0.0f;
-          }
-      }
+      if (vp_any_nonfinite(acc, padded || m >= M)) redo(mc);
     }
     const uint32_t row = KIND == kGemmForward ? vp_row_part(p, mc) : static_cast<uint32_t>(mc) * static_cast<uint32_t>(K);
 #pragma unroll
@@ -517,21 +535,29 @@ __global__ void __launch_bounds__((VpGw<VT, TILE>::kThreads)) vp_gw_kernel(const
     turn(ms + MS, buf1);  // past the slice's end: zeros
   }
   if constexpr (!bf) {
-    if (vp_any_nonfinite(acc, false)) {
+    if (vp_any_nonfinite(acc, false)) {  // the sums again as plain f32 products
+      uint32_t n[4], k[WC];  // the lane's runs of 4 rows n, its columns
 #pragma unroll
-      for (int j = 0; j < WC; ++j)
+      for (int g = 0; g < 4; ++g) n[g] = vp_col_part(p, min(n0 + wn + 8 * g + 4 * half, N - 4));
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const uint32_t k = static_cast<uint32_t>(min(k0 + wk + 32 * j + (lane & 31), K - 1));
-          const uint32_t n = vp_col_part(p, min(n0 + wn + 8 * (i >> 2) + 4 * half + (i & 3), N - 1));
-          float s = 0.0f;
-          for (int m = m_lo; m < m_hi; ++m) {
-            const float y = static_cast<const float*>(p.gvalue)[vp_row_part(p, m) + n];
-            s = fmaf(MASK && p.mask[m] != 0 ? 0.0f : y, static_cast<const float*>(p.x)[static_cast<uint32_t>(m) * static_cast<uint32_t>(K) + k], s);
-          }
-          acc[j].main[i] = s;
-          acc[j].small[i] = 0.0f;
+      for (int j = 0; j < WC; ++j) {
+        k[j] = static_cast<uint32_t>(min(k0 + wk + 32 * j + (lane & 31), K - 1));
+        acc[j].clear();
+      }
+#pragma unroll 4
+      for (int m = m_lo; m < m_hi; ++m) {
+        const float* y = static_cast<const float*>(p.gvalue) + vp_row_part(p, m);
+        const float* x = static_cast<const float*>(p.x) + static_cast<uint32_t>(m) * static_cast<uint32_t>(K);
+        const bool off = MASK && p.mask[m] != 0;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const vp_f4 v = *reinterpret_cast<const vp_f4*>(y + n[g]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < WC; ++j) acc[j].main[4 * g + i] = fmaf(off ? 0.0f : v[i], x[k[j]], acc[j].main[4 * g + i]);
         }
+      }
     }
   }
 #pragma unroll
