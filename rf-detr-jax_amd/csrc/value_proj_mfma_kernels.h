@@ -9,8 +9,8 @@
 // under the rounding of an f32 sum. Relative 2-norm against float64 at K = N = 256, 576 x 8 to 6800 x
 // 16 rows (v_mfma_f32_32x32x2_f32 in brackets): output 7e-8 (1.1e-7), grad_input 9e-8 (1.5e-7),
 // grad_weight 1.1e-7 to 2.5e-7 (1.6e-7 to 3.9e-7). The split turns an infinity (or a value that
-// rounds to one in bf16) into NaN, so a wave whose sums are not all finite computes its block again
-// in plain f32, runs of 8 columns and indices at a time: with an infinity in one row the 4608-row forward
+// rounds to one in bf16) into NaN, and of values below 2^-109 the third term leaves bf16's range, so a
+// wave with a sum that is not finite, or not zero and below 2^-105, computes its block again in plain f32, runs of 8 columns and indices at a time: with such a row the 4608-row forward
 // takes 61 us instead of 17, grad_weight 45 instead of 19, at 108800 rows 235 (94) and 397 (124), with one in
 // the weights, which every row meets, 88 and 1200. (One product at a time took 393 and 540 us, 893 and 3750,
 // 947 and 13300.)
@@ -92,14 +92,22 @@ struct VpAcc {
   __device__ __forceinline__ float at(int i) const { return main[i] + small[i]; }
 };
 
+// Whether a sum of the wave is not finite, or is below 2^-105 and not zero: operands that small have lost
+// their low bits (the third term of a value below 2^-109 leaves bf16's range).
+constexpr int kVpLeastLog2 = 105;
 template <int TERMS, int NB>
-__device__ __forceinline__ bool vp_any_nonfinite(const VpAcc<TERMS> (&acc)[NB], bool ignore) {
+__device__ __forceinline__ bool vp_any_lost(const VpAcc<TERMS> (&acc)[NB], bool ignore) {
   float s = 0.0f;
+  uint32_t least = 0xffffffffu;  // of (bits shifted past the sign) - 1, unsigned: a zero wraps to the largest
 #pragma unroll
   for (int j = 0; j < NB; ++j)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) s = fmaf(acc[j].at(i), 0.0f, s);
-  return __any(s != s && !ignore) != 0;
+    for (int i = 0; i < 16; ++i) {
+      const float v = acc[j].at(i);
+      s = fmaf(v, 0.0f, s);
+      least = min(least, (__float_as_uint(v) << 1) - 1u);
+    }
+  return __any((s != s || least < (static_cast<uint32_t>(127 - kVpLeastLog2) << 24) - 1u) && !ignore) != 0;
 }
 
 __device__ __forceinline__ float vp_sum8(const float (&f)[8]) {
@@ -326,7 +334,7 @@ __global__ void __launch_bounds__((VpRows<KIND, VT, CB>::kThreads)) vp_rows_kern
     const int m = tl * 32 + (lane & 31);
     const int mc = min(m, M - 1);
     if constexpr (!bf) {
-      if (vp_any_nonfinite(acc, padded || m >= M)) redo(mc);
+      if (vp_any_lost(acc, padded || m >= M)) redo(mc);
     }
     const uint32_t row = KIND == kGemmForward ? vp_row_part(p, mc) : static_cast<uint32_t>(mc) * static_cast<uint32_t>(K);
 #pragma unroll
@@ -535,7 +543,7 @@ __global__ void __launch_bounds__((VpGw<VT, TILE>::kThreads)) vp_gw_kernel(const
     turn(ms + MS, buf1);  // past the slice's end: zeros
   }
   if constexpr (!bf) {
-    if (vp_any_nonfinite(acc, false)) {  // the sums again as plain f32 products
+    if (vp_any_lost(acc, false)) {  // the sums again as plain f32 products
       uint32_t n[4], k[WC];  // the lane's runs of 4 rows n, its columns
 #pragma unroll
       for (int g = 0; g < 4; ++g) n[g] = vp_col_part(p, min(n0 + wn + 8 * g + 4 * half, N - 4));

@@ -342,3 +342,24 @@ def test_matrix_unit_kernels_nonfinite(tune, bf16):
         assert np.array_equal(np.isnan(a), np.isnan(ref)), name
         assert np.array_equal(a[~fine & ~np.isnan(ref)], ref[~fine & ~np.isnan(ref)]), name
         np.testing.assert_allclose(a[fine], ref[fine], rtol=2.0 ** -8 if bf16 else 1e-6, atol=0)
+
+
+@pytest.mark.parametrize("where", ["x", "w", "g"])
+@pytest.mark.parametrize("size", [1e-33, 1e-36])
+@pytest.mark.parametrize("blocks", [1, 2])
+def test_matrix_unit_kernels_of_tiny_tensors(tune, blocks, size, where):
+    """Results of values whose low bits leave bf16's range keep f32's precision: 1e-6 of the 2-norm, as
+    test_matrix_unit_kernels."""
+    rng = np.random.default_rng(38)
+    b, s, k, h, d = 3, 400, 72, 4, 24
+    t = {"x": rng.standard_normal((b, s, k)), "w": rng.standard_normal((h * d, k)), "g": rng.standard_normal((b * h, s, d))}
+    t[where] *= size
+    t["x"][1, 7:200] = 0.0  # sums of exactly zero need no second look
+    t = {n: a.astype(np.float32) for n, a in t.items()}
+    tune({"MSDA_VP_CB": blocks})
+    got = [value_proj_forward(_t(t["x"]), _t(t["w"]), None, h), *value_proj_backward(_t(t["x"]), _t(t["w"]), h, _t(t["g"]))[:2]]
+    torch.cuda.synchronize()
+    x, w, g = (t[n].astype(np.float64) for n in "xwg")
+    for name, a, ref in zip(("value", "grad_input", "grad_weight"), got, [VP.value_proj_rows(x, w, None, h), *VP.value_proj_rows_vjp(x, w, h, g)[:2]]):
+        err = np.linalg.norm(_np(a).astype(np.float64) - ref) / np.linalg.norm(ref)
+        assert err <= 1e-6, (name, err)
