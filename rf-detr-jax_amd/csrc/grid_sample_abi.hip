@@ -93,6 +93,7 @@ int msda_grid_sample_fwd(const void* input, int dtype, const float* grid, int gr
       const int lds = static_cast<int>(p.fwd_chunk * plane_bytes);
       // 16-byte copies when the input and every plane start on 16 bytes
       p.fwd_vec16 = aligned_to(input, 16) && plane_bytes % 16 == 0;
+      p.fwd_xcd = groups > n;  // a slice has several workgroups
       static std::atomic<int> granted_f[msda_host::kMaxDevices], granted_b[msda_host::kMaxDevices];
       if (dtype == MSDA_DTYPE_BF16) {
         if ((rc = msda_host::allow_lds(msda::gs_fwd_lds_kernel<msda::bf16_t>, lds, granted_b)) != MSDA_OK) return rc;
@@ -104,7 +105,12 @@ int msda_grid_sample_fwd(const void* input, int dtype, const float* grid, int gr
       return msda_host::check_launch("grid sample forward (staged)");
     }
   }
-  hipLaunchKernelGGL(msda::gs_fwd_kernel, dim3(lane_grid(static_cast<int64_t>(n) * n_points)), dim3(256), 0, st, p);
+  // A slice's workgroups on one XCD, but not where there are fewer than one a CU and each walks many bf16
+  // channels (10000 points a slice, 200x200: four slices of 256 channels 332 us in the order of dispatch, 393 on
+  // one XCD, of 64 channels 85 and 98, but of 16 24 and 13.5; f32 276 and 266; eight slices 534 and 538).
+  const int grid_size = lane_grid(static_cast<int64_t>(n) * n_points);
+  p.fwd_xcd = dtype != MSDA_DTYPE_BF16 || channels < 64 || grid_size >= cus;
+  hipLaunchKernelGGL(msda::gs_fwd_kernel, dim3(grid_size), dim3(256), 0, st, p);
   return msda_host::check_launch("grid sample forward");
 }
 

@@ -45,6 +45,7 @@ struct GridSampleParams {
   int fwd_chunk;          // gs_fwd_lds_kernel: channel planes staged per workgroup
   int fwd_split;          // gs_fwd_lds_kernel: workgroups sharing one (slice, chunk)'s points
   int fwd_vec16;          // gs_fwd_lds_kernel: the staged planes may be copied 16 bytes at a time
+  int fwd_xcd;            // forward: consecutive workgroups on one XCD, else in the order of dispatch
 };
 
 __device__ __forceinline__ float gs_load(const void* base, int64_t i, bool bf16) {
@@ -133,12 +134,12 @@ __device__ __forceinline__ GsCorners gs_corners(float gx, float gy, const GridSa
 // One lane per (slice, point); n * points < 2^31 (checked on the host), so indices are 32-bit. The
 // workgroups of a slice run on one XCD, so its planes are read into one L2 (in hardware order every
 // XCD with a workgroup of the slice reads the same cache lines): 400 one-channel 112x112 f32 planes,
-// 784 points each, 9.5 -> 4.8 us (nearest 4.9 -> 3.5).
+// 784 points each, 9.5 -> 4.8 us (nearest 4.9 -> 3.5). The host turns that off where it does not pay.
 __global__ void __launch_bounds__(256) gs_fwd_kernel(const GridSampleParams p) {
   const uint32_t total = static_cast<uint32_t>(p.n) * static_cast<uint32_t>(p.points);
   const int64_t plane = static_cast<int64_t>(p.h) * p.w;
   const bool bf = p.bf16 != 0;
-  const uint32_t block = static_cast<uint32_t>(xcd_logical(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x)));
+  const uint32_t block = p.fwd_xcd ? static_cast<uint32_t>(xcd_logical(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x))) : blockIdx.x;
   for (uint32_t i = block * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
     const uint32_t n32 = i / static_cast<uint32_t>(p.points);
     const int64_t n = n32;
@@ -167,22 +168,25 @@ constexpr int kGsAhead = 4;
 // planes (consecutive in [N, C, H, W]) are copied into LDS once in the input dtype (stage_copy:
 // global_load_lds_dwordx4 when rows allow 16-byte copies), then each lane samples its points from
 // LDS: the corner gathers of a wave touch random words, which from L2 would cost a cache line each.
-// Bound by the latency of its two reads, so the lane's first points are requested before the copy;
-// the workgroups of one slice are consecutive logical ids (xcd_logical), which share an L2.
-// 400 one-channel 112x112 f32 planes, 2352 points each: 11.8 -> 7.5 us.
+// Bound by the latency of its two reads, so an f32 lane's first points are requested before the copy
+// (400 one-channel 112x112 planes, 2352 points each: 8.1 -> 7.7 us; in bf16, where there are twice as many
+// waves a CU, that gained nothing: 16 x 256 channels of 100x160, 20000 points, 162 -> 175). The workgroups of one
+// slice are consecutive logical ids (xcd_logical), which share an L2, where it has several (f32, 112x112:
+// 11.8 -> 7.7; one a slice, 57x68 bf16 planes of 2412 points, 7.7 -> 7.9).
 template <typename VT>
 __global__ void __launch_bounds__(512) gs_fwd_lds_kernel(const GridSampleParams p) {
   extern __shared__ __align__(16) unsigned char gs_raw[];
   VT* plane_lds = reinterpret_cast<VT*>(gs_raw);
   const int nchunks = (p.c + p.fwd_chunk - 1) / p.fwd_chunk;
-  int id = xcd_logical(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
+  constexpr int AHEAD = std::is_same<VT, float>::value ? kGsAhead : 0;
+  int id = p.fwd_xcd ? xcd_logical(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x)) : static_cast<int>(blockIdx.x);
   const int share = id % p.fwd_split;
   id /= p.fwd_split;
   const int chunk = id % nchunks;
   const int n = id / nchunks;
   const int c0 = chunk * p.fwd_chunk, c1 = min(p.c, c0 + p.fwd_chunk);
   const int plane = p.h * p.w;
-  const bool bf = p.bf16 != 0;
+  constexpr bool bf = !std::is_same<VT, float>::value;
   const VT* src = static_cast<const VT*>(p.input) + (static_cast<int64_t>(n) * p.c + c0) * plane;
   const int per = (p.points + p.fwd_split - 1) / p.fwd_split;
   const int pt0 = share * per, pt1 = min(p.points, pt0 + per);
@@ -190,9 +194,9 @@ __global__ void __launch_bounds__(512) gs_fwd_lds_kernel(const GridSampleParams 
   // the lane's points are first + o, o = 0, step, 2 step .. < left (unsigned: no overflow at any count)
   const int first = pt0 + static_cast<int>(threadIdx.x);
   const uint32_t left = first < pt1 ? static_cast<uint32_t>(pt1 - first) : 0u, step = blockDim.x;
-  float2 ahead[kGsAhead];
+  float2 ahead[AHEAD + 1];
 #pragma unroll
-  for (int u = 0; u < kGsAhead; ++u) ahead[u] = u * step < left ? grid[first + u * step] : make_float2(0.0f, 0.0f);
+  for (int u = 0; u < AHEAD; ++u) ahead[u] = u * step < left ? grid[first + u * step] : make_float2(0.0f, 0.0f);
   stage_copy<VT>(plane_lds, src, (c1 - c0) * plane, p.fwd_vec16 != 0);
   __syncthreads();
   const MSDA_LDS VT* pl_all = (const MSDA_LDS VT*)(plane_lds);
@@ -210,13 +214,15 @@ __global__ void __launch_bounds__(512) gs_fwd_lds_kernel(const GridSampleParams 
       } else {
         v = ((rd(pl, k.c00) * k.w00 + rd(pl, k.c10) * k.w10) + rd(pl, k.c01) * k.w01) + rd(pl, k.c11) * k.w11;
       }
-      gs_store(p.out, (static_cast<int64_t>(n) * p.c + c) * p.points + pt, v, bf);
+      const int64_t at = (static_cast<int64_t>(n) * p.c + c) * p.points + pt;
+      if constexpr (bf) static_cast<__bf16*>(p.out)[at] = static_cast<__bf16>(v);  // v_cvt_pk_bf16_f32: nearest even, quiet NaN
+      else static_cast<float*>(p.out)[at] = v;
     }
   };
 #pragma unroll
-  for (int u = 0; u < kGsAhead; ++u)
+  for (int u = 0; u < AHEAD; ++u)
     if (u * step < left) sample(first + u * step, ahead[u]);
-  for (uint32_t o = kGsAhead * step; o < left; o += step) sample(first + o, grid[first + o]);
+  for (uint32_t o = AHEAD * step; o < left; o += step) sample(first + o, grid[first + o]);
 }
 
 // Workgroup = (slice n, channel chunk, row band); LDS: chunk x band_rows x W doubles. The sums are f64:
