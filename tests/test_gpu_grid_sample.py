@@ -208,3 +208,16 @@ def test_too_wide_for_the_accumulator_is_refused():
     with pytest.raises(Exception, match="width 16385"):
         hip.grid_sample_backward(v, torch.zeros((1, 1, 2), device=_dev()), torch.zeros((1, 1, 1), device=_dev()), 0, 0, 0,
                                  needs=(True, False))
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+@pytest.mark.parametrize("n,c,h,w,points", [
+    (2, 7, 30, 30, 20),        # grad_input by 256 threads: several channels, few points
+    (2, 9, 37, 52, 257),       # channel shares that differ by one, points past 256
+    (3, 1, 64, 64, 512),       # one channel, as many contributions as 256 threads take
+    (3, 1, 64, 64, 513),       # and one more
+    (4, 64, 150, 200, 300),    # gathered: fewer workgroups than compute units, many channels
+    (2, 64, 40, 41, 600),      # staged, a slice's workgroups on one XCD
+])
+def test_channel_shares_and_workgroup_sizes(n, c, h, w, points, bf16):
+    test_bands_chunks_and_many_points(n, c, h, w, points, bf16)
