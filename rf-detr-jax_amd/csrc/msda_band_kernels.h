@@ -169,13 +169,15 @@ __device__ __forceinline__ void lds_add_f64(uint32_t byte_addr, double v) {
 // LDS cycle met in the even, then in the odd chunks of their rows, in half of the bank groups. The
 // dot is the sum of the two chunks' dots, the same in either order. Backward with this and sum_lanes,
 // eight images, 16 heads of 16, f32: one 24x24 level, 3900 queries x 2 points, 38.6 -> 37.4 us; 80x80 +
-// 20x20, 300 x 4 points (here with the order of items too), 49.8 -> 44.7.
-template <typename VT, int CH>
-constexpr bool band_swap() { return std::is_same<VT, float>::value && CH == 8; }
+// 20x20, 300 x 4 points (here with the order of items too), 49.8 -> 44.7. Only with head_dim 16 and 32 (KD): at
+// head_dim 8, where a row is one lane's two chunks, it cost more than it saved (two images, 633 queries on 2x3,
+// 5x6, 10x13: 26.3 us without it and 27.6 with it), from 24 up it gains a hundredth.
+template <typename VT, int CH, int KD>
+constexpr bool band_swap() { return std::is_same<VT, float>::value && CH == 8 && KD != 0; }
 
-template <typename VT, int CH>
+template <typename VT, int CH, int KD>
 __device__ __forceinline__ float row_dot(const VT* rows, int at, int swap, const float (&g)[CH]) {
-  if constexpr (band_swap<VT, CH>()) {
+  if constexpr (band_swap<VT, CH, KD>()) {
     const int first = at + 4 * swap;  // at is a multiple of 8
     float u[4], v[4];
     load_vec_lds<VT, 4>(rows + first, u);
@@ -197,9 +199,9 @@ __device__ __forceinline__ float row_dot(const VT* rows, int at, int swap, const
   }
 }
 
-template <typename VT, int CH>
+template <typename VT, int CH, int KD>
 __device__ __forceinline__ void swap_chunks(float (&g)[CH], int swap) {
-  if constexpr (band_swap<VT, CH>()) {
+  if constexpr (band_swap<VT, CH, KD>()) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const float lo = g[k], hi = g[4 + k];
@@ -209,13 +211,13 @@ __device__ __forceinline__ void swap_chunks(float (&g)[CH], int swap) {
   }
 }
 
-template <typename VT, int CH>
+template <typename VT, int CH, int KD>
 __device__ __forceinline__ void band_dots(const VT* rows, const Bilinear& c, int rel, int swap, const float (&g)[CH], float& d00, float& d10,
                                           float& d01, float& d11) {
-  d00 = row_dot<VT, CH>(rows, c.o00 - rel, swap, g);
-  d10 = row_dot<VT, CH>(rows, c.o10 - rel, swap, g);
-  d01 = row_dot<VT, CH>(rows, c.o01 - rel, swap, g);
-  d11 = row_dot<VT, CH>(rows, c.o11 - rel, swap, g);
+  d00 = row_dot<VT, CH, KD>(rows, c.o00 - rel, swap, g);
+  d10 = row_dot<VT, CH, KD>(rows, c.o10 - rel, swap, g);
+  d01 = row_dot<VT, CH, KD>(rows, c.o01 - rel, swap, g);
+  d11 = row_dot<VT, CH, KD>(rows, c.o11 - rel, swap, g);
 }
 
 // Sum over the `lps` consecutive lanes of a sample: neighbours by DPP (quad_perm [1, 0, 3, 2], then
@@ -453,11 +455,13 @@ __global__ void __launch_bounds__(kBandMaxThreads) bwd_band_kernel(const BandPar
       const Bilinear c = bilinear(xy[i].x, xy[i].y, L, D);
       if (want_dots && c.cy0 >= r0 && c.cy0 < r1) {
         float d00, d10, d01, d11;
-        band_dots<VT, CH>(vrows, c, rel - c0, sl & 1, g, d00, d10, d01, d11);
-        d00 = sum_lanes(d00, lps);
-        d10 = sum_lanes(d10, lps);
-        d01 = sum_lanes(d01, lps);
-        d11 = sum_lanes(d11, lps);
+        band_dots<VT, CH, KD>(vrows, c, rel - c0, sl & 1, g, d00, d10, d01, d11);
+        if (lps > 1) {  // head_dim 8 bf16, 16 images, 365 queries on four small levels: 22.9 us without this test, 21.0 with
+          d00 = sum_lanes(d00, lps);
+          d10 = sum_lanes(d10, lps);
+          d01 = sum_lanes(d01, lps);
+          d11 = sum_lanes(d11, lps);
+        }
         if (j == 0) {
           const float da = c.w00 * d00 + c.w10 * d10 + c.w01 * d01 + c.w11 * d11;
           const float g00 = c.m00 * d00, g10 = c.m10 * d10, g01 = c.m01 * d01, g11 = c.m11 * d11;
@@ -478,7 +482,7 @@ __global__ void __launch_bounds__(kBandMaxThreads) bwd_band_kernel(const BandPar
     float g[CH], gr[CH];
     load_grad(q, g);
     const bool gfin = want_dv ? rotate_grad(g, gr) : true;
-    swap_chunks<VT, CH>(g, sl & 1);
+    swap_chunks<VT, CH, KD>(g, sl & 1);
     for (int p0 = 0; p0 < P; p0 += PB) {
       float2 xy[PB];
       float a[PB];
@@ -567,7 +571,7 @@ __global__ void __launch_bounds__(kBandMaxThreads) bwd_band_kernel(const BandPar
       if (e < count) {
         float gr[CH];
         const bool gfin = want_dv ? rotate_grad(g, gr) : true;
-        swap_chunks<VT, CH>(g, sl & 1);
+        swap_chunks<VT, CH, KD>(g, sl & 1);
         if constexpr (FZ) {
           // the row's softmax weights (softmax_regs' operations) and locations (fused_location_at)
           float m = -__builtin_inff(), sum = 0.0f;
