@@ -85,6 +85,8 @@ def attention_forward(q, k, v, lay, strides_of, mask=None, drop=None):
     """``(out, stats)``; ``out`` is allocated like ``q``'s logical shape, contiguous. ``drop``:
     ``(rate, seed)`` for dropout on the weights, or None."""
     _check(q, k, v)
+    if k.dtype != q.dtype or v.dtype != q.dtype:
+        raise TypeError(f"q, k and v must be of one type, got {q.dtype}, {k.dtype}, {v.dtype}")
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     stats = torch.empty((lay.batch * lay.groups * lay.heads * lay.len * 4,), dtype=torch.float32, device=q.device)
     strides = (ctypes.c_int64 * 16)(*(strides_of(q) + strides_of(k) + strides_of(v) + strides_of(out)))
@@ -137,7 +139,13 @@ class _AttentionFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_out):
         q, k, v, out, stats, mask = ctx.saved_tensors
+        # hooks on saved tensors may hand back other types and layouts: as the kernels read them
+        q, k, v, out = (t if t.dtype == grad_out.dtype and t.stride(-1) == 1 else t.to(grad_out.dtype).contiguous() for t in (q, k, v, out))
+        stats = stats.to(torch.float32).contiguous()
         lay = ctx.lay
+        if any(t.shape != grad_out.shape for t in (q, k, v, out)) or stats.numel() != lay.batch * lay.groups * lay.heads * lay.len * 4:
+            raise ValueError("saved tensors came back with other shapes than they were saved")
+        _check(q, k, v, out, stats)
         strides_of = lay.strides_rows if ctx.rows else lay.strides_bhld
         gq, gk, gv = attention_backward(q, k, v, out, stats, grad_out, lay, strides_of, mask, ctx.needs_input_grad[:3], ctx.drop)
         return gq, gk, gv, None, None, None, None

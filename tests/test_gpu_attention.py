@@ -786,3 +786,35 @@ def test_split_backward_of_tiny_tensors(tune, where, length):
     _note(f"tiny {where} {length}: {errors}")
     for name, split, f32 in zip("qkv", *errors):
         assert split <= 2 * f32 + 2.0 ** -23, name
+
+
+def test_masked_attention_saved_tensor_hooks_and_types():
+    """The Python autograd function (mask or dropout): saved tensors that hooks hand back in another type or layout
+    reach the kernels by their values, other shapes and mixed input types are refused."""
+    torch.manual_seed(4)
+    ins = [torch.randn(2, 2, 40, 32, device=_dev()) for _ in range(3)]
+    mask = torch.rand(40, 40, device=_dev()) < 0.2
+    g = torch.randn(2, 2, 40, 32, device=_dev())
+
+    def grads(unpack):
+        t = [x.clone().requires_grad_() for x in ins]
+        with torch.autograd.graph.saved_tensors_hooks(lambda x: x, unpack):
+            out = scaled_dot_product_attention(*t, mask)
+        return torch.autograd.grad(out, t, g)
+
+    def floats(f):
+        return lambda x: f(x) if x.dtype == torch.float32 else x
+
+    pairs = ((floats(lambda x: x.bfloat16()), floats(lambda x: x.bfloat16().float())),
+             (floats(lambda x: x.movedim(-1, 0).contiguous().movedim(0, -1)), lambda x: x))
+    for got, want in pairs:
+        for a, b in zip(grads(got), grads(want)):
+            assert a.dtype == b.dtype and torch.equal(a, b)
+    with pytest.raises(ValueError, match="other shapes"):
+        grads(floats(lambda x: x[..., :-4]))
+    for i in range(3):
+        mixed = [x.bfloat16() if j == i else x for j, x in enumerate(ins)]
+        with pytest.raises(TypeError, match="one type"):
+            scaled_dot_product_attention(*mixed, mask)
+        with pytest.raises(TypeError, match="one type"):
+            scaled_dot_product_attention(*mixed)
