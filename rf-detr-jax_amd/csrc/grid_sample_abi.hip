@@ -76,7 +76,7 @@ int msda_grid_sample_fwd(const void* input, int dtype, const float* grid, int gr
   if ((rc = msda_host::device_attrs(&lds_bytes, &cus)) != MSDA_OK) return rc;
   // Staged when one plane fits in a third of the LDS (three workgroups per CU) and there are enough
   // points per plane to pay for the copy (measured on MI355X, 400 one-channel 112x112 f32 planes:
-  // 2352 points 7.5 us staged against 9.8 gathered through L2, 784 points 4.8 gathered; bf16 planes,
+  // 2352 points 7.7 us staged against 9.8 gathered through L2, 784 points 4.8 gathered; bf16 planes,
   // 2352 points 7.3 against 12.5).
   const int budget = std::min(lds_bytes / 3, 64 * 1024);
   const int64_t plane_bytes = static_cast<int64_t>(height) * width * static_cast<int64_t>(eb);
