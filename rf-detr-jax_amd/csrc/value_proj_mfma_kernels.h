@@ -10,10 +10,11 @@
 // 16 rows (v_mfma_f32_32x32x2_f32 in brackets): output 7e-8 (1.1e-7), grad_input 9e-8 (1.5e-7),
 // grad_weight 1.1e-7 to 2.5e-7 (1.6e-7 to 3.9e-7). The split turns an infinity (or a value that
 // rounds to one in bf16) into NaN, and of values below 2^-109 the third term leaves bf16's range, so a
-// wave with a sum that is not finite, or not zero and below 2^-105, computes its block again in plain f32, runs of 8 columns and indices at a time: with such a row the 4608-row forward
-// takes 61 us instead of 17, grad_weight 45 instead of 19, at 108800 rows 235 (94) and 397 (124), with one in
-// the weights, which every row meets, 88 and 1200. (One product at a time took 393 and 540 us, 893 and 3750,
-// 947 and 13300.)
+// wave with a sum that is not finite, or not zero and below 2^-105, computes its block again in plain
+// f32, runs of 8 columns and indices at a time: with such a row the 4608-row forward takes 61 us instead
+// of 17, grad_weight 45 instead of 19, at 108800 rows 235 (94) and 397 (124), with one in the weights,
+// which every row meets, 88 and 1200. (One product at a time took 393 and 540 us, 893 and 3750, 947 and
+// 13300.)
 //
 // Measured (graph replays, 256 -> 16 x 16, us; v_mfma_f32 kernels before -> these):
 //   bf16 16 x 6800 rows: forward 207 -> 34, grad_input 221 -> 31, grad_weight and bias 219 -> 44
